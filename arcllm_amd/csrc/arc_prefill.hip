@@ -4,26 +4,19 @@
 //
 // A prompt of M <= 256 tokens at positions pos0 .. pos0+M-1 is processed as
 // matrices: per layer (8 launches)
-//   [q|k|v] = X [Wq|Wk|Wv]^T  (split-K partials, one launch)   k_pf_gemm_qkv
+//   [q|k|v] = X [Wq|Wk|Wv]^T  (split-K partials, one launch)   k_mm_qkv
 //   + bias, RoPE on q and k, q -> fp32, k and v -> fp16 cache  k_pf_qkv_epi
 //   causal GQA over the cache (positions <= own) -> X (fp16)    k_pf_attn
-//   H += X Wo^T, X = RMSNorm(H) (ffn norm)                      k_pf_gemm, k_pf_res_norm
-//   s = silu(X Wg^T) * (X Wu^T) -> fp16                         k_pf_gemm<SWIGLU>
-//   H += s Wd^T, X = RMSNorm(H) (next layer's attention norm)   k_pf_gemm, k_pf_res_norm
+//   H += X Wo^T, X = RMSNorm(H) (ffn norm)                      k_mm, k_pf_res_norm
+//   s = silu(X Wg^T) * (X Wu^T) -> fp16                         k_mm<SWIGLU>
+//   H += s Wd^T, X = RMSNorm(H) (next layer's attention norm)   k_mm, k_pf_res_norm
 // after the embedding and the first layer's attention norm (k_pf_embed,
 // k_pf_rmsnorm), then the output RMSNorm + LM head + argmax on the last row
 // only (the decode step's kernels), leaving the argmax as the next token.
 //
-// GEMM (pf_gemm_body): Y[m][n] = sum_k X[m][k] W[n][k] with
-// v_mfma_f32_32x32x16_f16.  A workgroup owns all M rows (MB blocks of 32) and
-// 128*NF weight rows (4 waves, NF rows per lane); X is staged through LDS in
-// half-super-block tiles (double-buffered, rows padded by 8 halves so the
-// 16-byte fragment reads are bank-conflict free); each lane dequantises its
-// own B fragments (8 weights of one row per 16-wide K step) straight from the
-// packed super-block into fp16 registers with the element decode's fp32
-// arithmetic, software-pipelined against the MFMAs.  Operands are fp16,
-// accumulation fp32.
+// GEMM: arc_pf_gemm.hpp (packed weights decoded in registers, X through LDS).  Operands are fp16, accumulation fp32.
 #include "arc_session.hpp"
+#include "arc_pf_gemm.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -33,656 +26,7 @@
 
 namespace arc {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // native vector: stays in registers
-
-constexpr int kPfKT = 128;         // K columns per LDS stage (half a super-block)
-constexpr int kPfLd = kPfKT + 8;   // padded LDS row, in halves
-
-// ------------------------------------------------------------------ GEMM
-struct PfGemm {
-    const uint8_t* w0;   // PLAIN: rows [0, ncol0); SWIGLU: gate
-    const uint8_t* w1;   // PLAIN: rows [ncol0, N) (row index - ncol0); SWIGLU: up
-    uint64_t row_bytes;
-    uint32_t ncol0;
-    uint32_t N;          // output columns
-    uint32_t nb;         // super-blocks per weight row
-    uint32_t bps;        // super-blocks per split (grid.y = splits)
-    uint32_t M;          // valid rows
-    uint32_t mpad;       // rows of the partial buffer per split
-    const _Float16* x;   // [>= MB*32 rows][ldx]
-    uint32_t ldx;
-    float* out;          // PLAIN: [split][mpad][ldo], columns [0, N)
-    uint32_t ldo;
-    uint32_t tiles;      // column tiles (workgroups along x) of this operand
-    _Float16* s;         // SWIGLU: [M][lds_out]
-    uint32_t lds_out;
-};
-
-// K order inside a super-block.  The GEMM sums over K, so X and W only have
-// to agree on which element each MFMA K slot holds.  Step t (0..7) of half
-// block hb gives the lane of half kh (lane / 32) the 8 consecutive elements
-// hb*128 + acol(t) + kh*16 .. +7, with acol(t) = (t/2)*32 + (t%2)*8, so one
-// lane's elements for a whole super-block come from a few contiguous 16-byte
-// pieces of the packed block:
-//   Q4_K: qs bytes c*32 + kh*16 .. +15 of chunk c hold elements
-//         c*64 + kh*16 + 0..15 (low nibbles) and c*64 + 32 + kh*16 + 0..15
-//         (high nibbles); steps t = 4(c%2) + r take the low nibbles of bytes
-//         0..7 (r=0) / 8..15 (r=1), the high nibbles of 0..7 (r=2) / 8..15 (r=3);
-//   Q6_K: ql bytes h*64 + 32*(q%2) + kh*16 .. +15 and qh bytes
-//         128 + h*32 + kh*16 .. +15 hold quarter q of half h, elements
-//         h*128 + q*32 + kh*16 + 0..15; step t = 2q + u takes bytes 8u .. 8u+7.
-__device__ __forceinline__ constexpr uint32_t acol(int t) { return uint32_t((t >> 1) * 32 + (t & 1) * 8); }
-
-// The packed bytes of one super-block row that one lane consumes, loaded a
-// super-block ahead of their use.
-template <int FMT>
-struct WRaw;
-template <>
-struct WRaw<kFmtQ4> {
-    u32x4 hdr;    // d, dmin, 12 scale bytes
-    u32x4 qs[4];  // qs chunk c, bytes kh*16 .. +15
-};
-template <>
-struct WRaw<kFmtQ6> {
-    u32x4 v[7];      // 16-byte pieces read from the dword floor: ql h*64 + {0,32} + kh*16 (h = 0, 1),
-    uint32_t e[7];   // qh 128 + h*32 + kh*16, scales 192; e = the dword after each piece
-    uint32_t d;      // bytes 208..209
-    uint32_t sh;     // block address mod 4 (0 or 2: Q6_K blocks are 210 bytes)
-};
-
-// The same bytes ready for the element decode, with the per-step factors
-// (codes are read as fp16 subnormals, q * 2^-24, so the factor carries
-// 2^24): Q4_K f[j] = d*sc_j * 2^24 (odd j: 2^20, as those steps read 16*q),
-// g[j] = -dmin*mn_j; Q6_K f[h*4 + q] = d*sc * 2^24 and n = -32*d*sc for
-// sc = sc_{h*8 + 2q + kh}, this lane's 16-element sub-block of quarter q.
-template <int FMT>
-struct WDec;
-template <>
-struct WDec<kFmtQ4> {
-    u32x4 qs[4];
-    float f[8], g[8];
-};
-template <>
-struct WDec<kFmtQ6> {
-    u32x4 ql[4], qh[2];
-    float f[8], n[8];
-};
-// Padded Q6_K (the model's Q6_K tensors): the same block bytes at a dword
-// boundary, so load_w reads them with sh = 0; only the block stride differs.
-template <>
-struct WRaw<kFmtQ6P> : WRaw<kFmtQ6> {};
-template <>
-struct WDec<kFmtQ6P> : WDec<kFmtQ6> {};
-template <int FMT>
-constexpr int pf_block_bytes()
-{
-    return FMT == kFmtQ4 ? kQ4Bytes : FMT == kFmtQ6P ? kQ6PBytes : kQ6Bytes;
-}
-
-template <int FMT>
-__device__ __forceinline__ void load_w(const uint8_t* blk, uint32_t kh, WRaw<FMT>& r)
-{
-    if constexpr (FMT == kFmtQ4) {
-        r.hdr = *reinterpret_cast<const u32x4*>(blk);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) r.qs[c] = *reinterpret_cast<const u32x4*>(blk + 16 + c * 32 + kh * 16);
-    } else if constexpr (FMT == kFmtQ6P) {
-        // padded block at a dword boundary: the pieces as they are
-#pragma unroll
-        for (int i = 0; i < 7; ++i) {
-            const uint32_t o = i < 4 ? uint32_t(i) * 32u + kh * 16u : i < 6 ? 128u + uint32_t(i - 4) * 32u + kh * 16u : 192u;
-            r.v[i] = *reinterpret_cast<const u32x4a4*>(blk + o);
-            r.e[i] = 0u;
-        }
-        r.d = *reinterpret_cast<const uint16_t*>(blk + 208);
-        r.sh = 0u;
-    } else {
-        // every dword read lies inside the 210-byte block: a piece at offset o
-        // reads [o - sh, o - sh + 20) when sh = 2 and [o, o + 16) plus the
-        // dword at o + 12 when sh = 0
-        const uint32_t sh = uint32_t(reinterpret_cast<uintptr_t>(blk)) & 3u;
-        const uint8_t* b = blk - sh;
-        const uint32_t eo = sh ? 16u : 12u;
-#pragma unroll
-        for (int i = 0; i < 7; ++i) {
-            const uint32_t o = i < 4 ? uint32_t(i) * 32u + kh * 16u : i < 6 ? 128u + uint32_t(i - 4) * 32u + kh * 16u : 192u;
-            r.v[i] = *reinterpret_cast<const u32x4a4*>(b + o);
-            r.e[i] = *reinterpret_cast<const uint32_t*>(b + o + eo);
-        }
-        r.d = *reinterpret_cast<const uint16_t*>(blk + 208);
-        r.sh = sh;
-    }
-}
-
-template <int FMT>
-__device__ __forceinline__ void decode_w(const WRaw<FMT>& r, uint32_t kh, WDec<FMT>& w)
-{
-#pragma clang fp contract(off)
-    if constexpr (FMT == kFmtQ4) {
-        const float d = f16_bits_to_f32(r.hdr.x), dmin = f16_bits_to_f32(r.hdr.x >> 16);
-        const float d24 = d * 16777216.0f, d20 = d * 1048576.0f;  // exact
-        const uint32_t b[3] = {r.hdr.y, r.hdr.z, r.hdr.w};
-        auto byte = [&](int i) { return (b[i >> 2] >> (8 * (i & 3))) & 0xffu; };
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            uint32_t sc, mn;
-            if (j < 4) {
-                sc = byte(j) & 63u;
-                mn = byte(j + 4) & 63u;
-            } else {
-                sc = (byte(j + 4) & 15u) | ((byte(j - 4) >> 6) << 4);
-                mn = (byte(j + 4) >> 4) | ((byte(j) >> 6) << 4);
-            }
-            w.f[j] = ((j & 1) ? d20 : d24) * float(sc);
-            w.g[j] = -(dmin * float(mn));
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) w.qs[c] = r.qs[c];
-        (void)kh;
-    } else {
-        u32x4 al[7];
-#pragma unroll
-        for (int i = 0; i < 7; ++i) {
-            if constexpr (FMT == kFmtQ6P) {
-                al[i] = r.v[i];
-                continue;
-            }
-            al[i].x = __builtin_amdgcn_alignbyte(r.v[i].y, r.v[i].x, r.sh);
-            al[i].y = __builtin_amdgcn_alignbyte(r.v[i].z, r.v[i].y, r.sh);
-            al[i].z = __builtin_amdgcn_alignbyte(r.v[i].w, r.v[i].z, r.sh);
-            al[i].w = __builtin_amdgcn_alignbyte(r.e[i], r.v[i].w, r.sh);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w.ql[i] = al[i];
-        w.qh[0] = al[4];
-        w.qh[1] = al[5];
-        const float d = f16_bits_to_f32(r.d);
-        const uint32_t s = 8u * kh;
-        const uint32_t sw[4] = {al[6].x >> s, al[6].y >> s, al[6].z >> s, al[6].w >> s};
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const float f = d * float(int8_t(uint8_t(sw[h * 2 + (q >> 1)] >> (16 * (q & 1)))));
-                w.f[h * 4 + q] = f * 16777216.0f;
-                w.n[h * 4 + q] = f * -32.0f;
-            }
-    }
-}
-
-// Two codes held in the low bits of the fp16 halves of `pair` read as exact
-// subnormals (bits c -> c * 2^-24); fmaf(code * 2^-24, A, n) with A the
-// element factor times 2^24 is v_fma_mix.
-__device__ __forceinline__ float mixc(uint32_t pair, bool hi, float A, float n)
-{
-    const half2_t h = __builtin_bit_cast(half2_t, pair);
-    return __builtin_fmaf(static_cast<float>(hi ? h.y : h.x), A, n);
-}
-
-__device__ __forceinline__ float opaque_f(float v)
-{
-    asm("" : "+v"(v));
-    return v;
-}
-
-// Four weights from the four bytes of `codes` (each code < 2^10, in the low
-// bits of its byte or, for Q4_K high nibbles, times 16): bytes 0 and 2 are
-// the halves of codes & 0x00ff00ff, bytes 1 and 3 moved down by v_perm_b32.
-// Each weight is the element decode's fp32 value rounded to fp16.  Left to
-// itself the compiler fuses the fp32 FMA and the fp16 conversion into one
-// v_fma_mix{lo,hi}_f16, which rounds the exact d*sc*q - dmin*mn to fp16
-// directly; for Q4_K that value can need more bits than fp32 holds, and
-// where its fp32 rounding is an fp16 tie the two roundings differ by an fp16
-// ulp.  ROUND32 keeps the fp32 value (the reference's weight) in a register
-// first.  Q6_K's d*sc*(q-32) is exact in fp32, so the fused form is the same.
-template <bool ROUND32>
-__device__ __forceinline__ void mix4w(uint32_t codes, float A, float n, half8& o, int at)
-{
-    const uint32_t ev = opaque(codes & 0x00ff00ffu);
-    const uint32_t od = opaque(__builtin_amdgcn_perm(0u, codes, 0x0c030c01u));  // [b1, 0, b3, 0]
-    float w[4] = {mixc(ev, false, A, n), mixc(od, false, A, n), mixc(ev, true, A, n), mixc(od, true, A, n)};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[at + i] = _Float16(ROUND32 ? opaque_f(w[i]) : w[i]);
-}
-
-// Step T of half HB: this lane's 8 weights as fp16, decoded in fp32 as one
-// fused multiply-add per element on the code read as an fp16 subnormal:
-// Q4_K fmaf(q * 2^-24, d*sc * 2^24, -dmin*mn) (high nibbles: 16q * 2^-24
-// against d*sc * 2^20), Q6_K fmaf((q+32) * 2^-24, d*sc * 2^24, -32*d*sc)
-// with q+32 the stored 6-bit code.  The scalings by powers of two are exact,
-// and both equal the element decode's (d*sc)*q - dmin*mn and (d*sc)*(q-32)
-// bit for bit: d has 11 significant bits, sc at most 6 (Q4_K) or 7 (Q6_K)
-// and q at most 4 or 6, so the product is exact in fp32 and only the final
-// add rounds.
-template <int FMT, int HB, int T>
-__device__ __forceinline__ half8 dequant_step(const WDec<FMT>& w)
-{
-    half8 o;
-    if constexpr (FMT == kFmtQ4) {
-        constexpr int c = HB * 2 + (T >> 2), r = T & 3, j = 2 * c + (r >> 1);
-        constexpr uint32_t mask = r < 2 ? 0x0f0f0f0fu : 0xf0f0f0f0u;
-        const float A = w.f[j], n = w.g[j];
-        mix4w<true>(w.qs[c][(r & 1) * 2] & mask, A, n, o, 0);
-        mix4w<true>(w.qs[c][(r & 1) * 2 + 1] & mask, A, n, o, 4);
-    } else {
-        constexpr int q = T >> 1, u = T & 1;
-        constexpr uint32_t lsh = (q >> 1) * 4u, hsh = q * 2u;
-        const u32x4& l = w.ql[HB * 2 + (q & 1)];
-        const u32x4& hh = w.qh[HB];
-        const uint32_t c0 = ((l[2 * u] >> lsh) & 0x0f0f0f0fu) | (((hh[2 * u] >> hsh) & 0x03030303u) << 4);
-        const uint32_t c1 = ((l[2 * u + 1] >> lsh) & 0x0f0f0f0fu) | (((hh[2 * u + 1] >> hsh) & 0x03030303u) << 4);
-        const float A = w.f[HB * 4 + q], n = w.n[HB * 4 + q];
-        mix4w<false>(c0, A, n, o, 0);
-        mix4w<false>(c1, A, n, o, 4);
-    }
-    return o;
-}
-
-// X staging of one LDS stage: K columns [k0, k0+128) of rows [0, MB*32),
-// MB*32*16 pieces of 16 bytes, MB*2 per thread, moved in two parts of MB
-// pieces (part P: pieces P*MB .. P*MB + MB-1 of each thread).  Piece i of a
-// thread is row (tid/16) + 16*i, columns (tid%16)*8 .. +7: the global loads
-// are buffer loads with the lane's byte offset `voff` and the uniform row and
-// column offset in a scalar register; the LDS stores use one base and
-// immediate offsets.
-struct XSrc {
-    __amdgpu_buffer_rsrc_t rsrc;  // X, MB*32 rows of ldx fp16
-    uint32_t voff;                // ((tid/16)*ldx + (tid%16)*8) * 2
-    uint32_t ldx;
-};
-
-template <int MB, int P>
-__device__ __forceinline__ void x_fetch(const XSrc& xs, uint32_t k0, u32x4 (&reg)[MB])
-{
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-        const uint32_t soff = (16u * uint32_t(P * MB + i) * xs.ldx + k0) * 2u;
-        reg[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xs.rsrc, xs.voff, soff, 0));
-    }
-}
-
-template <int MB, int P>
-__device__ __forceinline__ void x_store(_Float16* stage, const u32x4 (&reg)[MB])
-{
-    _Float16* base = stage + (P * MB * 16) * kPfLd + (threadIdx.x >> 4) * kPfLd + (threadIdx.x & 15u) * 8u;
-#pragma unroll
-    for (int i = 0; i < MB; ++i) *reinterpret_cast<u32x4*>(base + i * 16 * kPfLd) = reg[i];
-}
-
-template <int MB>
-__device__ __forceinline__ void load_a(const _Float16* a, half8 (&f)[MB])
-{
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) f[mb] = *reinterpret_cast<const half8*>(a + mb * 32 * kPfLd);
-}
-
-// Workgroup barrier ordering LDS only: global loads in flight (the next
-// super-block's weights, the next X stage) stay in flight across it.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// Per-lane state of the GEMM pipeline: NF B fragments (weight rows) per
-// lane against MB A fragments (32-row blocks of X).
-template <int FMT, int MB, int NF>
-struct PfState {
-    f32x16 acc[NF][MB];
-    half8 af[MB];          // A fragments of the step being issued
-    WDec<FMT> dec[NF];     // the current super-block, decoded
-    WRaw<FMT> raw[NF];     // the next super-block, as loaded
-};
-
-// Step T of half HB.  The NF*MB MFMAs of this step (B fragments `bc`, A
-// fragments in s.af) issue one A block at a time; right behind each block's
-// MFMAs its A fragment for step T+1 is read from LDS into the same registers,
-// and the B fragments of the next step are decoded into `bn` in between.  At
-// T = 7 the next step is step 0 of the next half: half 1 of this super-block,
-// or, once s.raw is decoded into s.dec, half 0 of the next super-block (its A
-// fragments are read after the barrier).  The sched_group_barrier pattern
-// keeps MFMA, LDS read and VALU interleaved so one wave per SIMD keeps the
-// matrix pipe busy.
-template <int FMT, int MB, int NF, int HB, int T>
-__device__ __forceinline__ void pf_step(PfState<FMT, MB, NF>& s, const _Float16* a, uint32_t kh, const half8 (&bc)[NF],
-                                        half8 (&bn)[NF])
-{
-    constexpr bool kNextSb = T == 7 && HB == 1;
-    if constexpr (kNextSb) {
-#pragma unroll
-        for (int j = 0; j < NF; ++j) decode_w<FMT>(s.raw[j], kh, s.dec[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < NF; ++j) bn[j] = dequant_step<FMT, (T == 7 ? 1 - HB : HB), (T + 1) & 7>(s.dec[j]);
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-        for (int j = 0; j < NF; ++j)
-            s.acc[j][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(s.af[mb], bc[j], s.acc[j][mb], 0, 0, 0);
-        if constexpr (T < 7) s.af[mb] = *reinterpret_cast<const half8*>(a + acol(T + 1) + mb * 32 * kPfLd);
-    }
-    constexpr int kValu = ((kNextSb ? 110 : 34) * NF + MB - 1) / MB;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-        __builtin_amdgcn_sched_group_barrier(0x008, NF, 0);  // MFMA
-        if constexpr (T < 7) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-        __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);  // VALU
-    }
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// One half super-block of MFMAs from LDS stage `a`, while the other stage
-// (not read during this half) is filled with K columns [xk0, xk0+128) of X
-// in two parts.  Half 1 also issues the weight loads of the next super-block
-// (after the first X part, so that waiting for X never waits for them); they
-// are decoded in its last step.  b0 holds the B fragments of step 0 on entry
-// and of the next half's step 0 on exit.
-template <int FMT, int MB, int NF, int HB>
-__device__ __forceinline__ void pf_half(const XSrc& p, PfState<FMT, MB, NF>& s, const _Float16* a, uint32_t xk0,
-                                        _Float16* xdst, const uint8_t* const (&wnext)[NF], uint32_t kh,
-                                        half8 (&b0)[NF], half8 (&b1)[NF])
-{
-    u32x4 xr[MB];
-    x_fetch<MB, 0>(p, xk0, xr);
-    if constexpr (HB == 1) {
-#pragma unroll
-        for (int j = 0; j < NF; ++j) load_w<FMT>(wnext[j], kh, s.raw[j]);
-    }
-    load_a<MB>(a, s.af);
-    __builtin_amdgcn_sched_barrier(0);
-    pf_step<FMT, MB, NF, HB, 0>(s, a, kh, b0, b1);
-    pf_step<FMT, MB, NF, HB, 1>(s, a, kh, b1, b0);
-    pf_step<FMT, MB, NF, HB, 2>(s, a, kh, b0, b1);
-    pf_step<FMT, MB, NF, HB, 3>(s, a, kh, b1, b0);
-    x_store<MB, 0>(xdst, xr);
-    x_fetch<MB, 1>(p, xk0, xr);
-    __builtin_amdgcn_sched_barrier(0);
-    pf_step<FMT, MB, NF, HB, 4>(s, a, kh, b0, b1);
-    pf_step<FMT, MB, NF, HB, 5>(s, a, kh, b1, b0);
-    pf_step<FMT, MB, NF, HB, 6>(s, a, kh, b0, b1);
-    pf_step<FMT, MB, NF, HB, 7>(s, a, kh, b1, b0);
-    x_store<MB, 1>(xdst, xr);
-}
-
-// D[m][c]: register i of block mb holds row mb*32 + (i/4)*8 + (lane/32)*4 + i%4
-__device__ __forceinline__ uint32_t acc_row(int mb, int i, int lane)
-{
-    return uint32_t(mb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3));
-}
-
-// ------------------------------------------ gate/up + SwiGLU in 8 waves
-// The fused gate/up GEMM with one weight row per lane (NF = 1): waves 0-3
-// own the tile's 128 gate rows, waves 4-7 its 128 up rows.  A wave then
-// needs half the accumulators of the NF = 2 layout, so two waves fit per
-// SIMD and one wave's dequantisation overlaps the other's MFMAs; every
-// weight is still dequantised once.  Each wave group stages one part of
-// every X tile (threads t & 255 of group g move part g), and SwiGLU is
-// joined through LDS at the end: the gate waves store silu(g) by
-// (row, column), the up waves multiply.
-// Pieces part*MB + sub*NP + i (i < NP, sub*NP + i < MB) of thread t & 255,
-// NP = ceil(MB / 2): each group moves its part in two halves.
-template <int MB>
-constexpr int gu_np()
-{
-    return (MB + 1) / 2;
-}
-
-template <int MB>
-__device__ __forceinline__ void x_fetch_part(const XSrc& xs, uint32_t k0, uint32_t part, int sub,
-                                             u32x4 (&reg)[gu_np<MB>()])
-{
-    constexpr int NP = gu_np<MB>();
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-        if (sub * NP + i >= MB) break;
-        const uint32_t soff = (16u * (part * MB + uint32_t(sub * NP + i)) * xs.ldx + k0) * 2u;
-        reg[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xs.rsrc, xs.voff, soff, 0));
-    }
-}
-
-template <int MB>
-__device__ __forceinline__ void x_store_part(_Float16* stage, uint32_t part, int sub, const u32x4 (&reg)[gu_np<MB>()])
-{
-    constexpr int NP = gu_np<MB>();
-    const uint32_t t = threadIdx.x & 255u;
-    _Float16* base = stage + (part * MB * 16) * kPfLd + (t >> 4) * kPfLd + (t & 15u) * 8u;
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-        if (sub * NP + i >= MB) break;
-        *reinterpret_cast<u32x4*>(base + (sub * NP + i) * 16 * kPfLd) = reg[i];
-    }
-}
-
-template <int FMT, int MB, int HB>
-__device__ __forceinline__ void pf_half_gu(const XSrc& p, PfState<FMT, MB, 1>& s, const _Float16* a, uint32_t xk0,
-                                           _Float16* xdst, const uint8_t* const (&wnext)[1], uint32_t kh, uint32_t part,
-                                           half8 (&b0)[1], half8 (&b1)[1])
-{
-    u32x4 xr[gu_np<MB>()];
-    x_fetch_part<MB>(p, xk0, part, 0, xr);
-    if constexpr (HB == 1) load_w<FMT>(wnext[0], kh, s.raw[0]);
-    load_a<MB>(a, s.af);
-    __builtin_amdgcn_sched_barrier(0);
-    pf_step<FMT, MB, 1, HB, 0>(s, a, kh, b0, b1);
-    pf_step<FMT, MB, 1, HB, 1>(s, a, kh, b1, b0);
-    pf_step<FMT, MB, 1, HB, 2>(s, a, kh, b0, b1);
-    pf_step<FMT, MB, 1, HB, 3>(s, a, kh, b1, b0);
-    x_store_part<MB>(xdst, part, 0, xr);
-    x_fetch_part<MB>(p, xk0, part, 1, xr);
-    __builtin_amdgcn_sched_barrier(0);
-    pf_step<FMT, MB, 1, HB, 4>(s, a, kh, b0, b1);
-    pf_step<FMT, MB, 1, HB, 5>(s, a, kh, b1, b0);
-    pf_step<FMT, MB, 1, HB, 6>(s, a, kh, b0, b1);
-    pf_step<FMT, MB, 1, HB, 7>(s, a, kh, b1, b0);
-    x_store_part<MB>(xdst, part, 1, xr);
-}
-
-template <int FMT, int MB>
-__global__ __launch_bounds__(512, 1) void k_pf_gemm_gu(PfGemm p)
-{
-    extern __shared__ __align__(16) _Float16 ash[];  // [2][MB*32][kPfLd]
-    constexpr int kStage = MB * 32 * kPfLd;
-    constexpr int kBB = pf_block_bytes<FMT>();
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t part = uint32_t(wave) >> 2, kh = uint32_t(lane) >> 5;
-    const uint32_t c = uint32_t(wave & 3) * 32 + uint32_t(lane & 31);  // column within the tile
-    const uint32_t col = blockIdx.x * 128 + c;
-    const uint8_t* wrow = (part == 0 ? p.w0 : p.w1) + uint64_t(min(col, p.N - 1)) * p.row_bytes;
-
-    PfState<FMT, MB, 1> s;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s.acc[0][mb][i] = 0.0f;
-
-    XSrc xs;
-    xs.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(p.x), (short)0, int(MB * 32 * p.ldx * 2u),
-                                                0x00020000);
-    const uint32_t t = uint32_t(tid) & 255u;
-    xs.voff = ((t >> 4) * p.ldx + (t & 15u) * 8u) * 2u;
-    xs.ldx = p.ldx;
-
-    // prologue: weights of super-block 0, stage 0 = half 0 of super-block 0
-    load_w<FMT>(wrow, kh, s.raw[0]);
-    {
-        u32x4 xr[gu_np<MB>()];
-        x_fetch_part<MB>(xs, 0, part, 0, xr);
-        x_store_part<MB>(ash, part, 0, xr);
-        x_fetch_part<MB>(xs, 0, part, 1, xr);
-        x_store_part<MB>(ash, part, 1, xr);
-    }
-    half8 b0[1], b1[1];
-    decode_w<FMT>(s.raw[0], kh, s.dec[0]);
-    b0[0] = dequant_step<FMT, 0, 0>(s.dec[0]);
-    lds_barrier();
-    const uint32_t ao = (lane & 31) * kPfLd + kh * 16;
-    const _Float16* a0 = ash + ao;
-    const _Float16* a1 = ash + opaque(ao + kStage);
-    for (uint32_t kb = 0; kb < p.nb; ++kb) {
-        const uint32_t kn = kb + 1 < p.nb ? kb + 1 : kb;  // the last super-block re-loads and re-stages itself
-        const uint8_t* wn[1] = {wrow + uint64_t(kn) * kBB};
-        pf_half_gu<FMT, MB, 0>(xs, s, a0, kb * kQK + kPfKT, ash + kStage, wn, kh, part, b0, b1);
-        lds_barrier();
-        pf_half_gu<FMT, MB, 1>(xs, s, a1, kn * kQK, ash, wn, kh, part, b0, b1);
-        lds_barrier();
-    }
-
-    // SwiGLU across the wave groups: silu(gate) by (row, column) in the free stages
-    float* sg = reinterpret_cast<float*>(ash);  // [MB*32][128]
-    if (part == 0) {
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float g = s.acc[0][mb][i];
-                sg[acc_row(mb, i, lane) * 128 + c] = g / (1.0f + expf(-g));
-            }
-    }
-    __syncthreads();
-    if (part == 1 && col < p.N) {
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const uint32_t m = acc_row(mb, i, lane);
-                if (m < p.M) p.s[uint64_t(m) * p.lds_out + col] = _Float16(sg[m * 128 + c] * s.acc[0][mb][i]);
-            }
-    }
-}
-
-// Y = X W^T over super-blocks [kb0, kb1) of K for MB*32 rows of X.
-// Workgroup: 4 waves, one per SIMD; lane (l%32) of wave w owns weight row(s)
-//   SWIGLU (NF = 2): gate and up row c = tile*128 + w*32 + l%32, and
-//                    writes s[m][c] = silu(X Wg^T)[m][c] * (X Wu^T)[m][c];
-//   PLAIN:           rows c_j = tile*128*NF + w*32*NF + j*32 + l%32
-//                    (row c < ncol0 from w0, else row c - ncol0 of w1), and
-//                    writes split partials out[blockIdx.y][m][c] (row stride ldo).
-// X is staged in LDS half a super-block (128 K columns) at a time, double-
-// buffered; the weights of super-block kb+1 are loaded during kb.
-template <int FMT, int MB, int NF, bool SWIGLU>
-__device__ __forceinline__ void pf_gemm_body(const PfGemm& p, uint32_t tile)
-{
-    static_assert(!SWIGLU || NF == 2, "SwiGLU pairs a gate and an up row per lane");
-    extern __shared__ __align__(16) _Float16 ash[];  // [2][MB*32][kPfLd]
-    constexpr int kStage = MB * 32 * kPfLd;
-    constexpr int kBB = pf_block_bytes<FMT>();
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t kh = uint32_t(lane) >> 5;
-
-    uint32_t col[NF];
-    const uint8_t* wrow[NF];
-#pragma unroll
-    for (int j = 0; j < NF; ++j) {
-        if constexpr (SWIGLU) {
-            col[j] = tile * 128 + wave * 32 + (lane & 31);
-            wrow[j] = (j == 0 ? p.w0 : p.w1) + uint64_t(min(col[j], p.N - 1)) * p.row_bytes;
-        } else {
-            col[j] = tile * (128 * NF) + wave * (32 * NF) + j * 32 + (lane & 31);
-            const uint32_t r = min(col[j], p.N - 1);
-            wrow[j] = r < p.ncol0 ? p.w0 + uint64_t(r) * p.row_bytes : p.w1 + uint64_t(r - p.ncol0) * p.row_bytes;
-        }
-    }
-    const uint32_t kb0 = blockIdx.y * p.bps, kb1 = min(p.nb, kb0 + p.bps);
-
-    PfState<FMT, MB, NF> s;
-#pragma unroll
-    for (int j = 0; j < NF; ++j)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) s.acc[j][mb][i] = 0.0f;
-
-    XSrc xs;
-    xs.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(p.x), (short)0, int(MB * 32 * p.ldx * 2u),
-                                                0x00020000);
-    xs.voff = ((uint32_t(tid) >> 4) * p.ldx + (uint32_t(tid) & 15u) * 8u) * 2u;
-    xs.ldx = p.ldx;
-
-    // prologue: weights of kb0, stage 0 = half 0 of kb0
-#pragma unroll
-    for (int j = 0; j < NF; ++j) load_w<FMT>(wrow[j] + uint64_t(kb0) * kBB, kh, s.raw[j]);
-    {
-        u32x4 xr[MB];
-        x_fetch<MB, 0>(xs, kb0 * kQK, xr);
-        x_store<MB, 0>(ash, xr);
-        x_fetch<MB, 1>(xs, kb0 * kQK, xr);
-        x_store<MB, 1>(ash, xr);
-    }
-    half8 b0[NF], b1[NF];
-#pragma unroll
-    for (int j = 0; j < NF; ++j) {
-        decode_w<FMT>(s.raw[j], kh, s.dec[j]);
-        b0[j] = dequant_step<FMT, 0, 0>(s.dec[j]);
-    }
-    lds_barrier();
-    // stage 1's A base is a separate register (its offsets from stage 0 exceed
-    // the 16-bit LDS immediate)
-    const uint32_t ao = (lane & 31) * kPfLd + kh * 16;
-    const _Float16* a0 = ash + ao;
-    const _Float16* a1 = ash + opaque(ao + kStage);
-    for (uint32_t kb = kb0; kb < kb1; ++kb) {
-        // the last super-block of the range re-loads and re-stages itself
-        const uint32_t kn = kb + 1 < kb1 ? kb + 1 : kb;
-        const uint8_t* wn[NF];
-#pragma unroll
-        for (int j = 0; j < NF; ++j) wn[j] = wrow[j] + uint64_t(kn) * kBB;
-        pf_half<FMT, MB, NF, 0>(xs, s, a0, kb * kQK + kPfKT, ash + kStage, wn, kh, b0, b1);
-        lds_barrier();
-        pf_half<FMT, MB, NF, 1>(xs, s, a1, kn * kQK, ash, wn, kh, b0, b1);
-        lds_barrier();
-    }
-
-    // D[m][c]: register i of block mb holds row mb*32 + (i/4)*8 + (lane/32)*4 + i%4
-    if constexpr (SWIGLU) {
-        if (col[0] < p.N) {
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const uint32_t m = mb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-                    if (m < p.M) {
-                        const float g = s.acc[0][mb][i], u = s.acc[1][mb][i];
-                        p.s[uint64_t(m) * p.lds_out + col[0]] = _Float16((g / (1.0f + expf(-g))) * u);
-                    }
-                }
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < NF; ++j) {
-            if (col[j] >= p.N) continue;
-            float* o = p.out + uint64_t(blockIdx.y) * p.mpad * p.ldo + col[j];
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const uint32_t m = mb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-                    if (m < p.M) o[uint64_t(m) * p.ldo] = s.acc[j][mb][i];
-                }
-        }
-    }
-}
-
-template <int FMT, int MB, int NF, bool SWIGLU>
-__global__ __launch_bounds__(256, 1) void k_pf_gemm(PfGemm p)
-{
-    pf_gemm_body<FMT, MB, NF, SWIGLU>(p, blockIdx.x);
-}
-
-// The q|k (Q4_K) and v (format VF) projections of one layer in one launch:
-// tiles [0, qk.tiles) are q|k, the rest v; both write split partials into
-// one [split][mpad][hidden + 2*kv_dim] buffer (v after q|k).
-template <int MB, int VF>
-__global__ __launch_bounds__(256, 1) void k_pf_gemm_qkv(PfGemm qk, PfGemm v)
-{
-    if (blockIdx.x < qk.tiles)
-        pf_gemm_body<kFmtQ4, MB, 1, false>(qk, blockIdx.x);
-    else
-        pf_gemm_body<VF, MB, 1, false>(v, blockIdx.x - qk.tiles);
-}
 
 // --------------------------------------------------------- small kernels
 // H[m] = dequant(token_embd[tokens[m]]); grid (nb, M), element formula of
@@ -780,17 +124,19 @@ __global__ __launch_bounds__(256) void k_pf_qkv_epi(const float* __restrict__ pa
     }
 }
 
-// Fixed-order second pass of a split-K projection with the residual and
-// (NORM) the next RMSNorm: H[m][c] += sum_s part[s][m][c] (s in order), X[m] =
-// fp16((H[m] * inv) * w), inv = 1/sqrt(mean(H[m]^2) + eps).  Grid M, one row
+// Fixed-order second pass of a split-K projection with the residual (when
+// `res` is set, which may be h) and (NORM) the next RMSNorm: H[m][c] = res[m][c]
+// + sum_s part[s][m][c] (s in order), X[m] = fp16((H[m] * inv) * w),
+// inv = 1/sqrt(mean(H[m]^2) + eps).  Grid M, one row
 // per workgroup of 1024 threads; thread t owns columns t + 1024*k (k < KC,
 // n <= 1024*KC), and loads the partials of 8 splits at a time, all in flight,
 // before adding them in split order.
 constexpr int kResCols = 20;  // n <= 20480, the model limit on hidden
 template <bool NORM, int KC>
 __global__ __launch_bounds__(1024) void k_pf_res_norm(const float* __restrict__ part, uint32_t splits, uint32_t mpad,
-                                                      uint32_t n, float* __restrict__ h, const float* __restrict__ w,
-                                                      float eps, _Float16* __restrict__ x, uint32_t ldx)
+                                                      uint32_t n, const float* res, float* h,
+                                                      const float* __restrict__ w, float eps, _Float16* __restrict__ x,
+                                                      uint32_t ldx)
 {
     static_assert(KC >= 1 && KC <= kResCols, "columns per thread");
     constexpr uint32_t kBatch = 8;
@@ -822,7 +168,7 @@ __global__ __launch_bounds__(1024) void k_pf_res_norm(const float* __restrict__ 
     for (int k = 0; k < KC; ++k) {
         const uint32_t c = t + 1024u * k;
         if (c < n) {
-            a[k] = r[c] + a[k];
+            if (res) a[k] = res[uint64_t(m) * n + c] + a[k];
             r[c] = a[k];
             if constexpr (NORM) ss = __builtin_fmaf(a[k], a[k], ss);
         }
@@ -841,16 +187,18 @@ __global__ __launch_bounds__(1024) void k_pf_res_norm(const float* __restrict__ 
 
 template <bool NORM>
 void launch_res_norm(uint32_t M, hipStream_t st, const float* part, uint32_t splits, uint32_t mpad, uint32_t n,
-                     float* h, const float* w, float eps, _Float16* x, uint32_t ldx)
+                     const float* res, float* h, const float* w, float eps, _Float16* x, uint32_t ldx)
 {
     const uint32_t kc = (n + 1023u) / 1024u;
     if (kc <= 4)
-        hipLaunchKernelGGL((k_pf_res_norm<NORM, 4>), dim3(M), dim3(1024), 0, st, part, splits, mpad, n, h, w, eps, x, ldx);
+        hipLaunchKernelGGL((k_pf_res_norm<NORM, 4>), dim3(M), dim3(1024), 0, st, part, splits, mpad, n, res, h, w, eps, x,
+                           ldx);
     else if (kc <= 8)
-        hipLaunchKernelGGL((k_pf_res_norm<NORM, 8>), dim3(M), dim3(1024), 0, st, part, splits, mpad, n, h, w, eps, x, ldx);
+        hipLaunchKernelGGL((k_pf_res_norm<NORM, 8>), dim3(M), dim3(1024), 0, st, part, splits, mpad, n, res, h, w, eps, x,
+                           ldx);
     else
-        hipLaunchKernelGGL((k_pf_res_norm<NORM, kResCols>), dim3(M), dim3(1024), 0, st, part, splits, mpad, n, h, w, eps,
-                           x, ldx);
+        hipLaunchKernelGGL((k_pf_res_norm<NORM, kResCols>), dim3(M), dim3(1024), 0, st, part, splits, mpad, n, res, h, w,
+                           eps, x, ldx);
 }
 
 // Causal GQA for query row m (position pos0 + m) and kv head g: the HPK q
@@ -1190,101 +538,87 @@ namespace {
 constexpr uint32_t kPfTargetWgs = 256;
 thread_local int g_pf_attn_mfma = 1;  // 0: the VALU attention kernel (k_pf_attn)
 
-template <int FMT, int MB, int NF, bool SW>
-hipError_t launch_gemm_t(const PfGemm& p, uint32_t gx, uint32_t splits, hipStream_t st)
+// Tile of an M-row pass: every wave takes all of the pass's rows (MF blocks of
+// 32) and 32 weight rows, so each weight is decoded once.  Plain products take
+// 4 waves (128 weight rows; 256 workgroups of them ran 17 % faster than 128 of
+// 8 waves, 3.7 against 4.3 us per super-block at 256 rows), split over K to
+// about one workgroup per CU; the fused gate/up, not split, 8 past 64 rows (128
+// gate and 128 up rows: 148 workgroups for 18944 columns, where 4 waves would
+// leave 40 CUs with a second one).
+#define ARC_MM_ROWS(M, CALL) ((M) > 128 ? CALL(8) : (M) > 64 ? CALL(4) : (M) > 32 ? CALL(2) : CALL(1))
+constexpr uint32_t kMmCols = 128;  // weight rows per workgroup of a plain product
+
+template <int FMT, int MF, int WN, bool SW>
+hipError_t launch_mm_t(const PfGemm& p, uint32_t splits, hipStream_t st)
 {
-    const size_t lds = size_t(2) * MB * 32 * kPfLd * sizeof(_Float16);
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_gemm<FMT, MB, NF, SW>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
-    hipLaunchKernelGGL((k_pf_gemm<FMT, MB, NF, SW>), dim3(gx, splits), dim3(256), lds, st, p);
+    constexpr uint32_t cols = SW ? 16u * WN : 32u * WN;
+    hipLaunchKernelGGL((k_mm<FMT, MF, 1, 1, WN, SW>), dim3((p.N + cols - 1) / cols, splits), dim3(64 * WN), 0, st, p);
     return hipGetLastError();
 }
 
-template <int MB>
-hipError_t launch_gu_t(const PfGemm& p, uint32_t gx, hipStream_t st)
+hipError_t launch_gateup(const PfGemm& p, hipStream_t st)
 {
-    const size_t lds = size_t(2) * MB * 32 * kPfLd * sizeof(_Float16);
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_gemm_gu<kFmtQ4, MB>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
-    hipLaunchKernelGGL((k_pf_gemm_gu<kFmtQ4, MB>), dim3(gx), dim3(512), lds, st, p);
-    return hipGetLastError();
+#define ARC_MM_CALL(MF) (launch_mm_t<kFmtQ4, MF, (MF >= 4 ? 8 : 4), true>(p, 1, st))
+    return ARC_MM_ROWS(p.M, ARC_MM_CALL);
+#undef ARC_MM_CALL
 }
 
-hipError_t launch_gateup(const PfGemm& p, uint32_t mb, uint32_t gx, hipStream_t st)
+template <int FMT>
+hipError_t launch_gemm_f(const PfGemm& p, uint32_t splits, hipStream_t st)
 {
-    switch (mb) {
-    case 1: return launch_gu_t<1>(p, gx, st);
-    case 2: return launch_gu_t<2>(p, gx, st);
-    case 4: return launch_gu_t<4>(p, gx, st);
-    default: return launch_gu_t<8>(p, gx, st);
-    }
+#define ARC_MM_CALL(MF) (launch_mm_t<FMT, MF, 4, false>(p, splits, st))
+    return ARC_MM_ROWS(p.M, ARC_MM_CALL);
+#undef ARC_MM_CALL
 }
 
-template <int FMT, int NF, bool SW>
-hipError_t launch_gemm_mb(const PfGemm& p, uint32_t mb, uint32_t gx, uint32_t splits, hipStream_t st)
+hipError_t launch_gemm(int qtype, const PfGemm& p, uint32_t splits, hipStream_t st)
 {
-    switch (mb) {
-    case 1: return launch_gemm_t<FMT, 1, NF, SW>(p, gx, splits, st);
-    case 2: return launch_gemm_t<FMT, 2, NF, SW>(p, gx, splits, st);
-    case 4: return launch_gemm_t<FMT, 4, NF, SW>(p, gx, splits, st);
-    default: return launch_gemm_t<FMT, 8, NF, SW>(p, gx, splits, st);
-    }
+    return qtype == kFmtQ4 ? launch_gemm_f<kFmtQ4>(p, splits, st) : launch_gemm_f<kFmtQ6P>(p, splits, st);
 }
 
-template <int MB, int VF>
-hipError_t launch_qkv_t(const PfGemm& qk, const PfGemm& v, uint32_t splits, hipStream_t st)
+template <int VF, int MF>
+hipError_t launch_qkv_t(const PfGemm& q, const PfGemm& k, const PfGemm& v, uint32_t splits, hipStream_t st)
 {
-    const size_t lds = size_t(2) * MB * 32 * kPfLd * sizeof(_Float16);
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_gemm_qkv<MB, VF>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
-    hipLaunchKernelGGL((k_pf_gemm_qkv<MB, VF>), dim3(qk.tiles + v.tiles, splits), dim3(256), lds, st, qk, v);
+    hipLaunchKernelGGL((k_mm_qkv<VF, MF, 1, 1, 4>), dim3(q.tiles + k.tiles + v.tiles, splits), dim3(256), 0, st, q, k, v);
     return hipGetLastError();
 }
 
 template <int VF>
-hipError_t launch_qkv_mb(const PfGemm& qk, const PfGemm& v, uint32_t mb, uint32_t splits, hipStream_t st)
+hipError_t launch_qkv_f(const PfGemm& q, const PfGemm& k, const PfGemm& v, uint32_t splits, hipStream_t st)
 {
-    switch (mb) {
-    case 1: return launch_qkv_t<1, VF>(qk, v, splits, st);
-    case 2: return launch_qkv_t<2, VF>(qk, v, splits, st);
-    case 4: return launch_qkv_t<4, VF>(qk, v, splits, st);
-    default: return launch_qkv_t<8, VF>(qk, v, splits, st);
-    }
+#define ARC_MM_CALL(MF) (launch_qkv_t<VF, MF>(q, k, v, splits, st))
+    return ARC_MM_ROWS(q.M, ARC_MM_CALL);
+#undef ARC_MM_CALL
 }
 
-hipError_t launch_qkv(const PfGemm& qk, const PfGemm& v, int vtype, uint32_t mb, uint32_t splits, hipStream_t st)
+uint32_t mm_tiles(uint32_t N)
 {
-    return vtype == kFmtQ4 ? launch_qkv_mb<kFmtQ4>(qk, v, mb, splits, st) : launch_qkv_mb<kFmtQ6P>(qk, v, mb, splits, st);
+    return (N + kMmCols - 1) / kMmCols;
 }
 
-uint32_t m_blocks(uint32_t M)
+// The q|k|v launch: operands q, k, v of the columns [0, H), [H, H + kvd),
+// [H + kvd, H + 2 kvd) of one partial buffer.
+hipError_t launch_qkv(PfGemm q, const uint8_t* wk, const uint8_t* wv, int vtype, uint32_t kvd, uint32_t splits, hipStream_t st)
 {
-    const uint32_t b = (M + 31) / 32;
-    return b <= 1 ? 1 : b <= 2 ? 2 : b <= 4 ? 4 : 8;
+    const uint32_t H = q.N;
+    q.tiles = mm_tiles(H);
+    PfGemm k = q, v = q;
+    k.w0 = wk;
+    k.out = q.out + H;
+    v.w0 = wv;
+    v.out = q.out + H + kvd;
+    k.N = v.N = kvd;
+    k.tiles = v.tiles = mm_tiles(kvd);
+    v.row_bytes = uint64_t(q.nb) * (vtype == kFmtQ4 ? kQ4Bytes : kQ6PBytes);
+    return vtype == kFmtQ4 ? launch_qkv_f<kFmtQ4>(q, k, v, splits, st) : launch_qkv_f<kFmtQ6P>(q, k, v, splits, st);
 }
 
-// Split-K plan of a PLAIN projection (NF = 1, 128 columns per workgroup):
-// the split count whose super-blocks per workgroup times rounds of
-// workgroups over the CUs (one resident workgroup per CU) is smallest, the
-// fewest splits (least partial traffic) among equals.
-void split_plan(uint32_t N, uint32_t nb, uint32_t& gx, uint32_t& splits, uint32_t& bps)
+// Split-K plan of a PLAIN projection of `gx` column tiles: the split count
+// whose super-blocks per workgroup times rounds of workgroups over the CUs
+// (one resident workgroup per CU) is smallest, the fewest splits (least
+// partial traffic) among equals.
+void split_plan(uint32_t gx, uint32_t nb, uint32_t& splits, uint32_t& bps)
 {
-    gx = (N + 127) / 128;
     uint32_t best = ~0u;
     for (uint32_t want = 1; want <= nb; ++want) {
         const uint32_t b = (nb + want - 1) / want, sp = (nb + b - 1) / b;
@@ -1295,6 +629,24 @@ void split_plan(uint32_t N, uint32_t nb, uint32_t& gx, uint32_t& splits, uint32_
             splits = sp;
         }
     }
+}
+
+void gemm_plan(uint32_t N, uint32_t nb, uint32_t& splits, uint32_t& bps)
+{
+    split_plan(mm_tiles(N), nb, splits, bps);
+}
+
+void qkv_plan(uint32_t H, uint32_t kvd, uint32_t nb, uint32_t& splits, uint32_t& bps)
+{
+    split_plan(mm_tiles(H) + 2 * mm_tiles(kvd), nb, splits, bps);
+}
+
+// Partials of an N-column projection: splits x 256 rows x N floats.
+uint64_t gemm_part_elems(uint32_t N, uint32_t nb)
+{
+    uint32_t sp, bps;
+    gemm_plan(N, nb, sp, bps);
+    return uint64_t(sp) * kPfMaxM * N;
 }
 
 template <int H>
@@ -1324,17 +676,9 @@ void launch_attn(uint32_t hpk, dim3 grid, hipStream_t st, const float* q, const 
 uint64_t prefill_part_elems(const arc_model_dims& d)
 {
     // q|k|v (one launch), o, down: [split][256][columns] partials
-    const uint32_t kvd = d.kv_heads * kHeadDim;
-    uint32_t gx, sp, bps;
-    uint64_t part = 0;
-    const uint32_t qkv_cols = ((d.hidden + kvd + 127) / 128 + (kvd + 127) / 128) * 128;
-    split_plan(qkv_cols, d.hidden / kQK, gx, sp, bps);
-    part = std::max(part, uint64_t(sp) * kPfMaxM * (d.hidden + 2 * kvd));
-    split_plan(d.hidden, d.hidden / kQK, gx, sp, bps);
-    part = std::max(part, uint64_t(sp) * kPfMaxM * d.hidden);
-    split_plan(d.hidden, d.ffn / kQK, gx, sp, bps);
-    part = std::max(part, uint64_t(sp) * kPfMaxM * d.hidden);
-    return part;
+    const uint32_t kvd = d.kv_heads * kHeadDim, nb = d.hidden / kQK;
+    return std::max({gemm_part_elems(d.hidden + 2 * kvd, nb), gemm_part_elems(d.hidden, nb),
+                     gemm_part_elems(d.hidden, d.ffn / kQK)});
 }
 
 int run_prefill(arc_session* S, const uint32_t* tokens, uint32_t n, uint32_t pos0, bool logits)
@@ -1357,7 +701,6 @@ int run_prefill(arc_session* S, const uint32_t* tokens, uint32_t n, uint32_t pos
     const float scale = 1.0f / std::sqrt(float(kHeadDim));
     for (uint32_t pass = 0; pass < passes; ++pass) {
         const uint32_t base = pass * kPfMaxM, M = std::min(uint32_t(kPfMaxM), n - base), p0 = pos0 + base;
-        const uint32_t mb = m_blocks(M);
         uint32_t* ht = pf->host_tokens + size_t(pass) * kPfMaxM;
         std::memcpy(ht, tokens + base, M * sizeof(uint32_t));
         if ((rc = check_hip(hipMemcpyAsync(pf->tokens, ht, M * sizeof(uint32_t), hipMemcpyHostToDevice, st), "tokens")))
@@ -1385,26 +728,16 @@ int run_prefill(arc_session* S, const uint32_t* tokens, uint32_t n, uint32_t pos
             g.ldx = H;
             g.nb = H / kQK;
             g.out = pf->part;
-            uint32_t gx, sp, bps;
+            uint32_t sp, bps;
             // q | k | v in one launch, partials [split][mpad][H | kvd | kvd]
             const uint32_t nqkv = H + 2 * kvd;
             g.w0 = L.q;
-            g.w1 = L.k;
             g.row_bytes = uint64_t(g.nb) * kQ4Bytes;
-            g.ncol0 = H;
-            g.N = H + kvd;
+            g.N = H;
             g.ldo = nqkv;
-            g.tiles = (g.N + 127) / 128;
-            PfGemm gv = g;
-            gv.w0 = gv.w1 = L.v;
-            gv.row_bytes = uint64_t(g.nb) * (L.v_type == kFmtQ4 ? kQ4Bytes : kQ6PBytes);
-            gv.ncol0 = kvd;
-            gv.N = kvd;
-            gv.out = pf->part + (H + kvd);
-            gv.tiles = (kvd + 127) / 128;
-            split_plan(g.tiles * 128 + gv.tiles * 128, g.nb, gx, sp, bps);
-            g.bps = gv.bps = bps;
-            if ((rc = chk(launch_qkv(g, gv, L.v_type, mb, sp, st), "q/k/v projection"))) return rc;
+            qkv_plan(H, kvd, g.nb, sp, bps);
+            g.bps = bps;
+            if ((rc = chk(launch_qkv(g, L.k, L.v, L.v_type, kvd, sp, st), "q/k/v projection"))) return rc;
             hipLaunchKernelGGL(k_pf_qkv_epi, dim3((nqkv / 2 + 255) / 256, M), dim3(256), 0, st, pf->part, sp,
                                uint32_t(kPfMaxM), H, kvd, L.qb, L.kb, L.vb, S->rope, p0, pf->q, kc, vc);
             if ((rc = chk(hipGetLastError(), "q/k/v epilogue"))) return rc;
@@ -1416,15 +749,14 @@ int run_prefill(arc_session* S, const uint32_t* tokens, uint32_t n, uint32_t pos
                 launch_attn(hpk, dim3(M, d.kv_heads), st, pf->q, kc, vc, d.kv_heads, p0, scale, pf->x, H);
             if ((rc = chk(hipGetLastError(), "prefill attention"))) return rc;
             // o + residual + ffn norm
-            g.w0 = g.w1 = L.o;
+            g.w0 = L.o;
             g.row_bytes = uint64_t(g.nb) * kQ4Bytes;
-            g.ncol0 = H;
             g.N = H;
             g.ldo = H;
-            split_plan(g.N, g.nb, gx, sp, bps);
+            gemm_plan(g.N, g.nb, sp, bps);
             g.bps = bps;
-            if ((rc = chk(launch_gemm_mb<kFmtQ4, 1, false>(g, mb, gx, sp, st), "o projection"))) return rc;
-            launch_res_norm<true>(M, st, pf->part, sp, uint32_t(kPfMaxM), H, pf->h, L.ffn_norm, d.rms_eps, pf->x, H);
+            if ((rc = chk(launch_gemm(kFmtQ4, g, sp, st), "o projection"))) return rc;
+            launch_res_norm<true>(M, st, pf->part, sp, uint32_t(kPfMaxM), H, pf->h, pf->h, L.ffn_norm, d.rms_eps, pf->x, H);
             if ((rc = chk(hipGetLastError(), "o residual + ffn norm"))) return rc;
             // gate/up + SwiGLU -> xs
             PfGemm u = g;
@@ -1432,32 +764,28 @@ int run_prefill(arc_session* S, const uint32_t* tokens, uint32_t n, uint32_t pos
             u.w1 = L.up;
             u.row_bytes = uint64_t(g.nb) * kQ4Bytes;
             u.N = F;
-            u.ncol0 = F;
             u.bps = g.nb;
             u.s = pf->xs;
             u.lds_out = F;
-            if ((rc = chk(launch_gateup(u, mb, (F + 127) / 128, st), "gate/up"))) return rc;
+            if ((rc = chk(launch_gateup(u, st), "gate/up"))) return rc;
             // down + residual (+ the next layer's attention norm)
             PfGemm dn = g;
             dn.x = pf->xs;
             dn.ldx = F;
             dn.nb = F / kQK;
-            dn.w0 = dn.w1 = L.down;
+            dn.w0 = L.down;
             dn.row_bytes = uint64_t(dn.nb) * (L.down_type == kFmtQ4 ? kQ4Bytes : kQ6PBytes);
-            dn.ncol0 = H;
             dn.N = H;
             dn.ldo = H;
-            split_plan(dn.N, dn.nb, gx, sp, bps);
+            gemm_plan(dn.N, dn.nb, sp, bps);
             dn.bps = bps;
-            rc = chk(L.down_type == kFmtQ4 ? launch_gemm_mb<kFmtQ4, 1, false>(dn, mb, gx, sp, st)
-                                           : launch_gemm_mb<kFmtQ6P, 1, false>(dn, mb, gx, sp, st),
-                     "down projection");
+            rc = chk(launch_gemm(L.down_type == kFmtQ4 ? kFmtQ4 : kFmtQ6P, dn, sp, st), "down projection");
             if (rc) return rc;
             if (l + 1 < d.layers) {
-                launch_res_norm<true>(M, st, pf->part, sp, uint32_t(kPfMaxM), H, pf->h, Mdl->layers[l + 1].attn_norm,
+                launch_res_norm<true>(M, st, pf->part, sp, uint32_t(kPfMaxM), H, pf->h, pf->h, Mdl->layers[l + 1].attn_norm,
                                       d.rms_eps, pf->x, H);
             } else {
-                launch_res_norm<false>(M, st, pf->part, sp, uint32_t(kPfMaxM), H, pf->h, nullptr, 0.0f, nullptr, 0u);
+                launch_res_norm<false>(M, st, pf->part, sp, uint32_t(kPfMaxM), H, pf->h, pf->h, nullptr, 0.0f, nullptr, 0u);
             }
             if ((rc = chk(hipGetLastError(), "down residual"))) return rc;
         }
@@ -1480,17 +808,15 @@ struct PfWorkspace {
     size_t x, part, bytes;
 };
 
-// X staging (256 rows of K fp16: the GEMM tiles read up to 256 rows) and the
-// split partials of the N x K projection's plan.
+// X staging (256 rows of K fp16, for rows at odd addresses) and the split
+// partials of the N x K projection's plan.
 PfWorkspace pf_workspace(uint32_t N, uint32_t K)
 {
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    uint32_t gx, sp, bps;
-    split_plan(N, K / kQK, gx, sp, bps);
     PfWorkspace w{};
     w.x = 0;
     w.part = up(size_t(kPfMaxM) * K * sizeof(_Float16));
-    w.bytes = w.part + up(size_t(sp) * kPfMaxM * N * sizeof(float));
+    w.bytes = w.part + up(size_t(gemm_part_elems(N, K / kQK)) * sizeof(float));
     return w;
 }
 
@@ -1507,24 +833,22 @@ int pf_check(const void* w, uint32_t N, uint32_t K, const uint16_t* x, uint32_t 
     return ARC_OK;
 }
 
-// Copies the M given rows of X into the staging area and zeroes the rows the
-// tiles read past them (up to the 32-row block count of M).
-int pf_stage_x(uint8_t* ws, const PfWorkspace& w, const uint16_t* x, uint32_t M, uint32_t K, hipStream_t st)
+// The GEMM's X: the given rows, or, where they do not start at a 16-byte
+// boundary (the tiles read 16 bytes at a time), a copy of them in the workspace.
+int pf_stage_x(uint8_t* ws, const PfWorkspace& w, const uint16_t* x, uint32_t M, uint32_t K, hipStream_t st, PfGemm& g)
 {
-    _Float16* xs = reinterpret_cast<_Float16*>(ws + w.x);
-    const size_t row = size_t(K) * sizeof(_Float16), rows = size_t(m_blocks(M)) * 32;
-    int rc = check_hip(hipMemcpyAsync(xs, x, M * row, hipMemcpyDeviceToDevice, st), "x staging");
-    if (rc) return rc;
-    if (rows > M) rc = check_hip(hipMemsetAsync(reinterpret_cast<uint8_t*>(xs) + M * row, 0, (rows - M) * row, st), "x pad");
-    return rc;
+    g.ldx = K;
+    g.x = reinterpret_cast<const _Float16*>(x);
+    if ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) return ARC_OK;
+    g.x = reinterpret_cast<const _Float16*>(ws + w.x);
+    return check_hip(hipMemcpyAsync(ws + w.x, x, size_t(M) * K * sizeof(_Float16), hipMemcpyDeviceToDevice, st), "x staging");
 }
 
 // y[m][c] = sum over the splits of part[s][m][c], in split order.
 int pf_reduce(const float* part, uint32_t splits, uint32_t M, uint32_t N, float* y, hipStream_t st)
 {
-    int rc = check_hip(hipMemsetAsync(y, 0, size_t(M) * N * sizeof(float), st), "y clear");
-    if (rc) return rc;
-    launch_res_norm<false>(M, st, part, splits, uint32_t(kPfMaxM), N, y, nullptr, 0.0f, nullptr, 0u);
+    launch_res_norm<false>(M, st, part, splits, uint32_t(kPfMaxM), N, nullptr, y, nullptr, 0.0f, nullptr,
+                           0u);
     return check_hip(hipGetLastError(), "split reduction");
 }
 
@@ -1558,27 +882,19 @@ int arc_prefill_gemm(int qtype, const void* w, uint32_t N, uint32_t K, const uin
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     const PfWorkspace pw = pf_workspace(N, K);
-    if ((rc = pf_stage_x(ws, pw, x, M, K, st))) return rc;
     PfGemm g{};
+    if ((rc = pf_stage_x(ws, pw, x, M, K, st, g))) return rc;
     g.M = M;
     g.mpad = kPfMaxM;
-    g.x = reinterpret_cast<const _Float16*>(ws + pw.x);
-    g.ldx = K;
     g.nb = K / kQK;
     g.out = reinterpret_cast<float*>(ws + pw.part);
-    g.w0 = g.w1 = static_cast<const uint8_t*>(w);
+    g.w0 = static_cast<const uint8_t*>(w);
     g.row_bytes = uint64_t(g.nb) * (qtype == kFmtQ4 ? kQ4Bytes : kQ6PBytes);
-    g.ncol0 = N;
     g.N = N;
     g.ldo = N;
-    uint32_t gx, sp, bps;
-    split_plan(N, g.nb, gx, sp, bps);
-    g.bps = bps;
-    const uint32_t mb = m_blocks(M);
-    rc = check_hip(qtype == kFmtQ4 ? launch_gemm_mb<kFmtQ4, 1, false>(g, mb, gx, sp, st)
-                                   : launch_gemm_mb<kFmtQ6P, 1, false>(g, mb, gx, sp, st),
-                   "prompt-pass GEMM");
-    if (rc) return rc;
+    uint32_t sp;
+    gemm_plan(N, g.nb, sp, g.bps);
+    if ((rc = check_hip(launch_gemm(qtype, g, sp, st), "prompt-pass GEMM"))) return rc;
     return pf_reduce(g.out, sp, M, N, y, st);
 }
 
@@ -1592,22 +908,19 @@ int arc_prefill_gateup(const void* w_gate, const void* w_up, uint32_t N, uint32_
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     const PfWorkspace pw = pf_workspace(N, K);
-    if ((rc = pf_stage_x(ws, pw, x, M, K, st))) return rc;
     PfGemm u{};
+    if ((rc = pf_stage_x(ws, pw, x, M, K, st, u))) return rc;
     u.M = M;
     u.mpad = kPfMaxM;
-    u.x = reinterpret_cast<const _Float16*>(ws + pw.x);
-    u.ldx = K;
     u.nb = K / kQK;
     u.w0 = static_cast<const uint8_t*>(w_gate);
     u.w1 = static_cast<const uint8_t*>(w_up);
     u.row_bytes = uint64_t(u.nb) * kQ4Bytes;
     u.N = N;
-    u.ncol0 = N;
     u.bps = u.nb;
     u.s = reinterpret_cast<_Float16*>(s);
     u.lds_out = N;
-    return check_hip(launch_gateup(u, m_blocks(M), (N + 127) / 128, st), "prompt-pass gate/up");
+    return check_hip(launch_gateup(u, st), "prompt-pass gate/up");
 }
 
 int arc_prefill_attention(const float* q, const void* kc, const void* vc, uint32_t kv_heads, uint32_t hpk,
@@ -1654,38 +967,22 @@ int arc_prefill_qkv(const void* wq, const void* wk, const void* wv, int v_qtype,
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     const PfWorkspace pw = pf_workspace(N, K);
-    if ((rc = pf_stage_x(ws, pw, x, M, K, st))) return rc;
-    // as run_prefill: q|k one operand, v the other, partials [split][mpad][H | kvd | kvd]
+    // as run_prefill: partials [split][mpad][H | kvd | kvd]
     PfGemm g{};
+    if ((rc = pf_stage_x(ws, pw, x, M, K, st, g))) return rc;
     g.M = M;
     g.mpad = kPfMaxM;
-    g.x = reinterpret_cast<const _Float16*>(ws + pw.x);
-    g.ldx = K;
     g.nb = K / kQK;
     g.out = reinterpret_cast<float*>(ws + pw.part);
     g.w0 = static_cast<const uint8_t*>(wq);
-    g.w1 = static_cast<const uint8_t*>(wk);
     g.row_bytes = uint64_t(g.nb) * kQ4Bytes;
-    g.ncol0 = H;
-    g.N = H + kvd;
+    g.N = H;
     g.ldo = N;
-    g.tiles = (g.N + 127) / 128;
-    PfGemm gv = g;
-    gv.w0 = gv.w1 = static_cast<const uint8_t*>(wv);
-    gv.row_bytes = uint64_t(g.nb) * (v_qtype == kFmtQ4 ? kQ4Bytes : kQ6PBytes);
-    gv.ncol0 = kvd;
-    gv.N = kvd;
-    gv.out = g.out + (H + kvd);
-    gv.tiles = (kvd + 127) / 128;
-    uint32_t gx, sp, bps;
-    split_plan(g.tiles * 128 + gv.tiles * 128, g.nb, gx, sp, bps);
-    g.bps = gv.bps = bps;
-    // the partial buffer is sized by the plan of N columns; the q|k|v plan's
-    // split count must fit it
-    uint32_t gx2, sp2, bps2;
-    split_plan(N, g.nb, gx2, sp2, bps2);
-    if (sp > sp2) return set_error(ARC_ERR_UNSUPPORTED, "internal: q/k/v split plan %u > workspace plan %u", sp, sp2);
-    if ((rc = check_hip(launch_qkv(g, gv, v_qtype, m_blocks(M), sp, st), "prompt-pass q/k/v"))) return rc;
+    uint32_t sp;
+    qkv_plan(H, kvd, g.nb, sp, g.bps);
+    rc = check_hip(launch_qkv(g, static_cast<const uint8_t*>(wk), static_cast<const uint8_t*>(wv), v_qtype, kvd, sp, st),
+                   "prompt-pass q/k/v");
+    if (rc) return rc;
     return pf_reduce(g.out, sp, M, N, y, st);
 }
 
