@@ -22,10 +22,12 @@
 // v_cvt_pk_f16_f32).  Each wave takes all rows of the pass (WM = 1), so a weight
 // is decoded once and feeds up to 8 MFMAs: 2.4 other vector instructions and
 // one LDS read (4 cycles of the LDS) per MFMA.  Gate/up 18944 x 3584 at 256 rows
-// (whole call): 87 us, 800 TFLOP/s, 100 us before (34 instructions to decode 8
+// (whole call): 79 us, 875 TFLOP/s, 100 us before (34 instructions to decode 8
 // weights, X through registers, two barriers' skew per super-block, a 30 KB
-// epilogue); at 100 rows 46 against 62; down 3584 x 18944 60 against 69; q|k|v at
-// 23 rows 12.8 against 18.6.  Tiles measured for the gate/up kernel alone: 32 x
+// epilogue); at 100 rows 43 against 62; down 3584 x 18944 57 against 69; q|k|v at
+// 23 rows 12.6 against 18.6.  The weights are loaded 12 steps ahead: with 8 (and
+// waited for together with X) weights from HBM cost 10 us more than weights from
+// the Infinity Cache (gate/up 89 against 79 us).  Tiles measured for the gate/up kernel alone: 32 x
 // 256 per wave, 8 waves 76-78 us; 64 x 128 (each weight decoded twice) 87; 48 x 128
 // and 48 x 256 with 16x16x32 77-78, 80 x 128 in 4 waves 78.
 //
@@ -70,8 +72,7 @@ constexpr int kMmKT = 128;             // K columns per LDS stage
 constexpr int kMmRowB = kMmKT * 2;     // bytes of a stage row
 
 // The bytes of one weight row's super-block that one lane consumes: the codes
-// of its two halves (each half is loaded into place as soon as the previous
-// super-block's is used up) and the scales as loaded ...
+// of its two halves and the scales as loaded ...
 template <int FMT>
 struct MmCodes;
 template <>
@@ -131,6 +132,20 @@ __device__ __forceinline__ void mm_load_codes(__amdgpu_buffer_rsrc_t w, uint32_t
         } else {
             r.ql[P][i] = mm_ld16(w, row + 32u * kh + (64u * P + 16u * i), blk);
             r.qh[P][i] = mm_ld16(w, row + (128u + 32u * P + 16u * i), blk);
+        }
+    }
+}
+
+template <int FMT, int P>
+__device__ __forceinline__ void mm_take(MmCodes<FMT>& to, const MmCodes<FMT>& from)
+{
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if constexpr (FMT == kFmtQ4) {
+            to.q[P][i] = from.q[P][i];
+        } else {
+            to.ql[P][i] = from.ql[P][i];
+            to.qh[P][i] = from.qh[P][i];
         }
     }
 }
@@ -276,7 +291,8 @@ struct Mm {
     f32x16 acc[NF][MF];
     half8 a[kD];
     half8 b[2][NF];
-    MmCodes<FMT> codes[NF];
+    MmCodes<FMT> codes[NF];     // in use
+    MmCodes<FMT> next[NF];      // in flight: 12 steps (about 3 us) from its load to its first use
     MmHdr<FMT> hdr[NF];
     MmScale<FMT> scale[NF];
     float fa[NF], fn[NF];
@@ -332,17 +348,18 @@ struct Mm {
         return *reinterpret_cast<const half8*>(stage + (frag ^ (mm_piece_step<FMT>(r) << 4)) + i * (32 * kMmRowB));
     }
 
-    // Half P of super-block kb's codes; its scales.
+    // Half P of super-block kb's codes, and with half 0 its scales: kLoads<P>
+    // load instructions.
     template <int P>
-    __device__ __forceinline__ void load_codes(uint32_t kb)
+    static constexpr int kLoads = NF * (FMT == kFmtQ4 ? 2 + (P == 0) : 4 + 2 * (P == 0));
+    template <int P>
+    __device__ __forceinline__ void load_w(uint32_t kb, MmCodes<FMT> (&c)[NF])
     {
 #pragma unroll
-        for (int f = 0; f < NF; ++f) mm_load_codes<FMT, P>(wr, wrow[f], kb * uint32_t(kBB), kh, codes[f]);
-    }
-    __device__ __forceinline__ void load_hdr(uint32_t kb)
-    {
-#pragma unroll
-        for (int f = 0; f < NF; ++f) mm_load_hdr<FMT>(wr, wrow[f], kb * uint32_t(kBB), hdr[f]);
+        for (int f = 0; f < NF; ++f) {
+            if constexpr (P == 0) mm_load_hdr<FMT>(wr, wrow[f], kb * uint32_t(kBB), hdr[f]);
+            mm_load_codes<FMT, P>(wr, wrow[f], kb * uint32_t(kBB), kh, c[f]);
+        }
     }
 
     // Weight fragments of step (P, R).
@@ -361,8 +378,10 @@ struct Mm {
     // super-block.  In front of fragment kSync the stage changes: from there on
     // `st` takes half P of kn, a quarter of the fill per step (issued together
     // right behind the barrier, every wave of the workgroup queued on the load
-    // path for about 1000 cycles), and half P of kn's codes is loaded (its
-    // fragments are made from the last step of the other half on).
+    // path for about 1000 cycles).  Half P of kn's codes is loaded in step 3,
+    // behind the last fill, so that the wait for the fills leaves it in flight
+    // (loads complete in issue order): its fragments are made from the last step
+    // of the other half on.
     template <int P, int R>
     __device__ __forceinline__ void step(uint8_t* st, uint8_t* ot, uint32_t kb, uint32_t kn)
     {
@@ -370,16 +389,20 @@ struct Mm {
         half8 (&bc)[NF] = b[R & 1];
         half8 (&bn)[NF] = b[1 - (R & 1)];
         if constexpr (R < 3) fill<R + 1>(ot, (P == 0 ? kb : kn) * 2u + (1 - P));
-        if constexpr (P == 1 && R == 0) load_hdr(kn);
+        if constexpr (R == 3) load_w<P>(kn, next);
+        if constexpr (R == 7) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) mm_take<FMT, kNextP>(codes[f], next[f]);
+        }
         make_b<kNextP, kNextR>(bn);
 #pragma unroll
         for (int i = 0; i < MF; ++i) {
             const int u = R * MF + i;
             if (u == kSync) {
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's fills of `ot`
+                // this wave's fills of `ot`; step 3's weight loads stay in flight
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads<P>) : "memory");
                 lds_barrier();
                 fill<0>(st, kn * 2u + P);
-                load_codes<P>(kn);
 #pragma unroll
                 for (int v = kUses - kD; v < kSync; ++v) a[v % kD] = frag_at(ot, (v + kD - kUses) / MF, (v + kD - kUses) % MF);
             }
@@ -410,9 +433,8 @@ struct Mm {
     // Super-blocks [kb0, kb1).
     __device__ __forceinline__ void run(uint8_t* s0, uint8_t* s1, uint32_t kb0, uint32_t kb1)
     {
-        load_hdr(kb0);
-        load_codes<0>(kb0);
-        load_codes<1>(kb0);
+        load_w<0>(kb0, codes);
+        load_w<1>(kb0, next);
         fill<0>(s0, kb0 * 2u);
         fill<1>(s0, kb0 * 2u);
         fill<2>(s0, kb0 * 2u);
