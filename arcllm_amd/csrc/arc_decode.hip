@@ -464,37 +464,56 @@ static Cfg dec_cfg(int kind, Cfg c)
 }
 
 template <int HPK, int W>
-static void launch_attn_hpk(const AttnParams& ap, uint32_t kv_heads, hipStream_t st)
+static void launch_attn_hpk(const AttnParams& ap, uint32_t nsplit, uint32_t kv_heads, hipStream_t st)
 {
     if (g_dry_run) return;
-    hipLaunchKernelGGL((k_attn<HPK, W>), dim3(kMaxSplits, kv_heads), dim3(W * kWave), 0, st, ap);
+    hipLaunchKernelGGL((k_attn<HPK, W>), dim3(nsplit, kv_heads), dim3(W * kWave), 0, st, ap);
 }
 
 template <int W>
-static void launch_attn_w(const AttnParams& ap, uint32_t kv_heads, hipStream_t st)
+static void launch_attn_w(const AttnParams& ap, uint32_t nsplit, uint32_t kv_heads, hipStream_t st)
 {
     switch (ap.hpk) {
-    case 1: launch_attn_hpk<1, W>(ap, kv_heads, st); break;
-    case 2: launch_attn_hpk<2, W>(ap, kv_heads, st); break;
-    case 3: launch_attn_hpk<3, W>(ap, kv_heads, st); break;
-    case 4: launch_attn_hpk<4, W>(ap, kv_heads, st); break;
-    case 5: launch_attn_hpk<5, W>(ap, kv_heads, st); break;
-    case 6: launch_attn_hpk<6, W>(ap, kv_heads, st); break;
-    case 7: launch_attn_hpk<7, W>(ap, kv_heads, st); break;
-    default: launch_attn_hpk<8, W>(ap, kv_heads, st); break;
+    case 1: launch_attn_hpk<1, W>(ap, nsplit, kv_heads, st); break;
+    case 2: launch_attn_hpk<2, W>(ap, nsplit, kv_heads, st); break;
+    case 3: launch_attn_hpk<3, W>(ap, nsplit, kv_heads, st); break;
+    case 4: launch_attn_hpk<4, W>(ap, nsplit, kv_heads, st); break;
+    case 5: launch_attn_hpk<5, W>(ap, nsplit, kv_heads, st); break;
+    case 6: launch_attn_hpk<6, W>(ap, nsplit, kv_heads, st); break;
+    case 7: launch_attn_hpk<7, W>(ap, nsplit, kv_heads, st); break;
+    default: launch_attn_hpk<8, W>(ap, nsplit, kv_heads, st); break;
     }
 }
 
-// Sets ap.min_cps and launches (grid: kMaxSplits x kv heads; workgroups past
-// the position's plan return at once).
-static void launch_attn(AttnParams ap, uint32_t kv_heads, hipStream_t st)
+// Sets ap.min_cps and launches.  T = 0: the position is only known on the
+// device (grid kMaxSplits x kv heads; workgroups past its plan return at once).
+// Otherwise the grid is the plan's, and the shape follows the context: the
+// merge reads every split's partials in one workgroup per kv head, so past 2048
+// positions half as many splits of 8 waves win, and past 4096, where 4 waves
+// take two chunks per split, two 8-wave chunks do for 4 kv heads or more (us per
+// call, 4 waves / 8 waves; kv heads x query heads per kv head):
+//   T = 2000  4x7 12.0 / 11.9   1x8 11.5 / 11.9   8x4 13.1 / 11.3   2x2  9.2 /  9.8
+//   T = 2500  4x7 13.6 / 12.8   1x8 12.7 / 12.6   8x4 14.7 / 12.1   2x2 10.1 / 10.0
+//   T = 4001  4x7 16.2 / 13.7   1x8 14.2 / 13.2   8x4 18.5 / 13.6   2x2 11.7 / 10.6
+//   T = 6000  4x7 16.6 / 15.9   1x8 15.0 / 16.1   8x4 17.2 / 14.5   2x2 11.9 / 12.6
+//   T = 8192  4x7 18.0 / 16.1   1x8 16.3 / 16.6   8x4 19.9 / 15.2   2x2 13.3 / 13.0
+static void launch_attn(AttnParams ap, uint32_t kv_heads, hipStream_t st, uint32_t T = 0)
 {
-    const int waves = g_attn_waves ? g_attn_waves : 4;
+    int waves = g_attn_waves ? g_attn_waves : 4;
     ap.min_cps = g_attn_min_cps > 0 ? uint32_t(g_attn_min_cps) : 1u;
+    if (!g_attn_waves && g_attn_min_cps <= 0) {
+        if (T > 4096 && kv_heads >= 4) {
+            waves = 8;
+            ap.min_cps = 2;
+        } else if (T > 2048 && T <= 4096) {
+            waves = 8;
+        }
+    }
+    const uint32_t nsplit = T ? attn_split(T, uint32_t(waves) * kAttnTile, ap.min_cps).nsplit : uint32_t(kMaxSplits);
     if (waves == 8)
-        launch_attn_w<8>(ap, kv_heads, st);
+        launch_attn_w<8>(ap, nsplit, kv_heads, st);
     else
-        launch_attn_w<4>(ap, kv_heads, st);
+        launch_attn_w<4>(ap, nsplit, kv_heads, st);
 }
 
 // Attention + o projection in one launch (k_attn_o): 1 automatic, 0 two
@@ -1458,7 +1477,7 @@ int arc_attention_decode(const float* q, const void* kc, const void* vc, uint32_
     ap.hpk = hpk;
     ap.max_ctx = max_ctx;
     ap.scale = 1.0f / std::sqrt(float(kHeadDim));
-    launch_attn(ap, kv_heads, st);
+    launch_attn(ap, kv_heads, st, T);
     return check_hip(hipGetLastError(), "attention");
 }
 
