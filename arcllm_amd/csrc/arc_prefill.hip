@@ -563,7 +563,8 @@ thread_local int g_pf_attn_mfma = 1;  // 0: the VALU attention kernel (k_pf_attn
 // about one workgroup per CU; the fused gate/up, not split, 8 past 64 rows (128
 // gate and 128 up rows: 148 workgroups for 18944 columns, where 4 waves would
 // leave 40 CUs with a second one).
-#define ARC_MM_ROWS(M, CALL) ((M) > 128 ? CALL(8) : (M) > 64 ? CALL(4) : (M) > 32 ? CALL(2) : CALL(1))
+#define ARC_MM_ROWS(M, CALL) \
+    ((M) > 192 ? CALL(8) : (M) > 128 ? CALL(6) : (M) > 96 ? CALL(4) : (M) > 64 ? CALL(3) : (M) > 32 ? CALL(2) : CALL(1))
 constexpr uint32_t kMmCols = 128;  // weight rows per workgroup of a plain product
 
 template <int FMT, int MF, int WN, bool SW>
@@ -576,7 +577,7 @@ hipError_t launch_mm_t(const PfGemm& p, uint32_t splits, hipStream_t st)
 
 hipError_t launch_gateup(const PfGemm& p, hipStream_t st)
 {
-#define ARC_MM_CALL(MF) (launch_mm_t<kFmtQ4, MF, (MF >= 4 ? 8 : 4), true>(p, 1, st))
+#define ARC_MM_CALL(MF) (launch_mm_t<kFmtQ4, MF, (MF >= 3 ? 8 : 4), true>(p, 1, st))
     return ARC_MM_ROWS(p.M, ARC_MM_CALL);
 #undef ARC_MM_CALL
 }

@@ -1,5 +1,5 @@
 """The prompt pass's tiled GEMM at the edges of its tiles: row counts around
-the 32 / 64 / 128 / 256-row tiles, column counts that are no multiple of a
+the 32 / 64 / 96 / 128 / 192 / 256-row tiles, column counts that are no multiple of a
 tile, a vector store or 8, and one and several splits of K; every row and
 column against the fp16-operand oracle.
 
@@ -38,7 +38,7 @@ def x16(M, K, stream, scale=1.0):
     return (arc.synth_normal(SEED, stream, M * K) * scale).astype(np.float16).reshape(M, K)
 
 
-@pytest.mark.parametrize("M", [1, 31, 32, 33, 64, 65, 127, 128, 129, 255, 256])
+@pytest.mark.parametrize("M", [1, 31, 32, 33, 64, 65, 96, 97, 127, 128, 129, 192, 193, 255, 256])
 @pytest.mark.parametrize("qtype,N,K", [(arc.Q4_K, 131, 2560), (arc.Q6_K_PADDED, 126, 256), (arc.Q6_K_PADDED, 257, 768)])
 def test_gemm_tile_edges(qtype, N, K, M):
     w, dw, oq = packed(qtype, N, K, 1 + N)
@@ -55,7 +55,7 @@ def test_gemm_tile_edges(qtype, N, K, M):
     assert not out[M * N:].any(), "wrote past the result"
 
 
-@pytest.mark.parametrize("M", [1, 32, 33, 65, 129, 256])
+@pytest.mark.parametrize("M", [1, 32, 33, 65, 96, 97, 129, 192, 193, 256])
 @pytest.mark.parametrize("N", [128, 200, 131])
 def test_gateup_tile_edges(N, M):
     K = 512
