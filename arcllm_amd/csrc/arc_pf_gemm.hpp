@@ -4,14 +4,20 @@
 //
 // Workgroup of WM x WN waves, wave (wm, wn) owns MF*32 rows of X and NF*32
 // weight rows with v_mfma_f32_32x32x16_f16 (lane l: X row / weight row l%32,
-// 8 of the 16 K elements by half-wave kh = l/32).  The K order is chosen so that
-// a lane's 8 elements of every step are whole dwords of the 16-byte pieces of
-// the packed block that it loads, and X is read from LDS in the same order:
-//   half block p (128 elements), step r of 8, half-wave kh:
-//   Q4_K: the 8 codes of nibble r>>2 of bytes 8(r&3) .. +7 of qs chunk 2p + kh,
-//         elements (2kh + (r>>2))*32 + 8(r&3) ..
-//   Q6_K: quarter q = kh + 2(r>>2), elements q*32 + 8(r&3) ..
-// so a lane needs the scales of half of the block's sub-blocks only.
+// 8 of the 16 K elements by half-wave kh = l/32).  The K order is the one that
+// every kernel of the prompt pass has summed in (half block p of 128 elements,
+// step r of 8, half-wave kh):
+//   elements p*128 + (r>>1)*32 + 16kh + 8(r&1) .. +7,
+// so that results stay the same bit for bit; X is read from LDS in the same
+// order.  Both formats hold a lane's 8 elements of a step in whole dwords of the
+// 16-byte pieces of the packed block that it loads:
+//   Q4_K: nibble (r>>1)&1 of bytes 16kh + 8(r&1) .. +7 of qs chunk 2p + (r>>2)
+//   Q6_K: quarter q = r>>1 of half p: ql bytes 64p + 32(q&1) + 16kh + 8(r&1) ..
+//         +7, nibble q>>1, and qh bytes 32p + 16kh + 8(r&1) .. +7, bits 2q, 2q + 1
+// (Half-wave kh on chunk 2p + kh or on quarter kh + 2(r>>2) would halve a lane's
+// Q4_K factors, but costs Q6_K a fourth load and shifts by kh, and measured no
+// faster: q|k|v at 23 rows 12.9 us against 12.5 here, down 56.4 against 55.5,
+// gate/up at 256 rows 74.0 against 74.9.)
 //
 // What bounds it: instruction issue, and at full size the chip's power (a
 // library fp16 product of 8192^3 runs at 1.23 PFLOP/s on this card, one of 256 x
@@ -77,12 +83,12 @@ template <int FMT>
 struct MmCodes;
 template <>
 struct MmCodes<kFmtQ4> {
-    u32x4 q[2][2];   // half p: qs bytes 64p + 32kh .. +31
+    u32x4 q[2][2];   // half p, chunk 2p + i: qs bytes 64p + 32i + 16kh .. +15
 };
 template <>
 struct MmCodes<kFmtQ6P> {
-    u32x4 ql[2][2];  // half h: ql bytes 64h + 32kh .. +31
-    u32x4 qh[2][2];  // half h: qh bytes 32h .. +31
+    u32x4 ql[2][2];  // half h: ql bytes 64h + 32i + 16kh .. +15
+    u32x4 qh[2];     // half h: qh bytes 32h + 16kh .. +15
 };
 template <int FMT>
 struct MmHdr;
@@ -100,12 +106,12 @@ template <int FMT>
 struct MmScale;
 template <>
 struct MmScale<kFmtQ4> {
-    uint32_t sc, mn;  // byte 2p + i: sub-block 4p + 2kh + i (steps 4i .. 4i+3 of half p)
-    float d24, dmin;  // d * 2^24
+    uint32_t sc[2], mn[2];  // half p, byte j: sub-block 4p + j (steps 2j, 2j + 1)
+    float d24, dmin;        // d * 2^24
 };
 template <>
 struct MmScale<kFmtQ6P> {
-    uint32_t sc[2];   // half h, byte 2i + j: quarter kh + 2i, its 16-element half j (steps 4i + 2j, +1)
+    uint32_t sc[2][2];  // half h, byte 2j of dword i: quarter 2i + j, its 16-element half kh (steps 2(2i + j), +1)
     float d;
 };
 template <int FMT>
@@ -125,15 +131,15 @@ template <int FMT, int P>
 __device__ __forceinline__ void mm_load_codes(__amdgpu_buffer_rsrc_t w, uint32_t row, uint32_t blk, uint32_t kh,
                                               MmCodes<FMT>& r)
 {
+    const uint32_t at = row + 16u * kh;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        if constexpr (FMT == kFmtQ4) {
-            r.q[P][i] = mm_ld16(w, row + 32u * kh + (16u + 64u * P + 16u * i), blk);
-        } else {
-            r.ql[P][i] = mm_ld16(w, row + 32u * kh + (64u * P + 16u * i), blk);
-            r.qh[P][i] = mm_ld16(w, row + (128u + 32u * P + 16u * i), blk);
-        }
+        if constexpr (FMT == kFmtQ4)
+            r.q[P][i] = mm_ld16(w, at + (16u + 64u * P + 32u * i), blk);
+        else
+            r.ql[P][i] = mm_ld16(w, at + (64u * P + 32u * i), blk);
     }
+    if constexpr (FMT != kFmtQ4) r.qh[P] = mm_ld16(w, at + (128u + 32u * P), blk);
 }
 
 template <int FMT, int P>
@@ -141,13 +147,12 @@ __device__ __forceinline__ void mm_take(MmCodes<FMT>& to, const MmCodes<FMT>& fr
 {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        if constexpr (FMT == kFmtQ4) {
+        if constexpr (FMT == kFmtQ4)
             to.q[P][i] = from.q[P][i];
-        } else {
+        else
             to.ql[P][i] = from.ql[P][i];
-            to.qh[P][i] = from.qh[P][i];
-        }
     }
+    if constexpr (FMT != kFmtQ4) to.qh[P] = from.qh[P];
 }
 
 template <int FMT>
@@ -165,40 +170,36 @@ template <int FMT>
 __device__ __forceinline__ void mm_unpack(const MmHdr<FMT>& r, uint32_t kh, MmScale<FMT>& c)
 {
     if constexpr (FMT == kFmtQ4) {
-        const uint32_t sh = 16u * kh;
-        const uint32_t yy = r.hdr.y >> sh, zz = r.hdr.z >> sh, ww = r.hdr.w >> sh;
-        c.sc = (yy & 0x3f3fu) | (((ww & 0x0f0fu) | ((yy >> 2) & 0x3030u)) << 16);
-        c.mn = (zz & 0x3f3fu) | ((((ww >> 4) & 0x0f0fu) | ((zz >> 2) & 0x3030u)) << 16);
+        c.sc[0] = r.hdr.y & 0x3f3f3f3fu;
+        c.sc[1] = (r.hdr.w & 0x0f0f0f0fu) | ((r.hdr.y >> 2) & 0x30303030u);
+        c.mn[0] = r.hdr.z & 0x3f3f3f3fu;
+        c.mn[1] = ((r.hdr.w >> 4) & 0x0f0f0f0fu) | ((r.hdr.z >> 2) & 0x30303030u);
         c.d24 = f16_bits_to_f32(r.hdr.x) * 16777216.0f;
         c.dmin = f16_bits_to_f32(r.hdr.x >> 16);
     } else {
-        // scale byte 8h + 2q + j, q = kh + 2i: bytes 2kh + j of scale dword 2h + i
-        const uint32_t sh = 16u * kh;
-        c.sc[0] = ((r.sc.x >> sh) & 0xffffu) | ((r.sc.y >> sh) << 16);
-        c.sc[1] = ((r.sc.z >> sh) & 0xffffu) | ((r.sc.w >> sh) << 16);
+        // scale byte 8h + 2q + kh, q = 2i + j: byte 2j + kh of scale dword 2h + i
+        const uint32_t sh = 8u * kh;
+        c.sc[0][0] = r.sc.x >> sh;
+        c.sc[0][1] = r.sc.y >> sh;
+        c.sc[1][0] = r.sc.z >> sh;
+        c.sc[1][1] = r.sc.w >> sh;
         c.d = f16_bits_to_f32(r.d);
     }
 }
 
-// Steps whose weights share one factor pair.
-template <int FMT>
-constexpr int mm_factor_steps()
-{
-    return FMT == kFmtQ4 ? 4 : 2;
-}
+constexpr int kMmFactorSteps = 2;  // steps whose weights share one factor pair
 
-// Factors of the steps from R on (R a multiple of mm_factor_steps) of half P:
+// Factors of the steps from R on (R a multiple of kMmFactorSteps) of half P:
 // weight = code * 2^-24 * a + n with the code read as an fp16 subnormal
 // (Q4_K high nibbles as 16 * code).
 template <int FMT, int P, int R>
 __device__ __forceinline__ void mm_factors(const MmScale<FMT>& c, float& a, float& n)
 {
     if constexpr (FMT == kFmtQ4) {
-        constexpr int i = 2 * P + (R >> 2);
-        a = ((R >> 2) ? c.d24 * 0.0625f : c.d24) * byte_f(c.sc, i);
-        n = -(c.dmin * byte_f(c.mn, i));
+        a = ((R & 2) ? c.d24 * 0.0625f : c.d24) * byte_f(c.sc[P], R >> 1);
+        n = -(c.dmin * byte_f(c.mn[P], R >> 1));
     } else {
-        const float f = c.d * float(int8_t(uint8_t(c.sc[P] >> (8 * (R >> 1)))));
+        const float f = c.d * float(int8_t(uint8_t(c.sc[P][R >> 2] >> (8 * (R & 2)))));
         a = f * 16777216.0f;
         n = f * -32.0f;
     }
@@ -228,23 +229,23 @@ __device__ __forceinline__ void mm_mix4(uint32_t ev, uint32_t od, float a, float
 
 // The lane's 8 weights of step R of half P.
 template <int FMT, int P, int R>
-__device__ __forceinline__ half8 mm_dequant(const MmCodes<FMT>& c, uint32_t kh, float a, float n)
+__device__ __forceinline__ half8 mm_dequant(const MmCodes<FMT>& c, float a, float n)
 {
     half8 o;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        constexpr int piece = (R & 3) >> 1;  // of the half's two 16-byte pieces
         const int dw = 2 * (R & 1) + k;
         uint32_t ev, od;
         if constexpr (FMT == kFmtQ4) {
-            constexpr uint32_t m = R < 4 ? 0x000f000fu : 0x00f000f0u;
-            ev = opaque(c.q[P][piece][dw] & m);
-            od = opaque((c.q[P][piece][dw] >> 8) & m);
+            constexpr uint32_t m = (R & 2) ? 0x00f000f0u : 0x000f000fu;
+            ev = opaque(c.q[P][R >> 2][dw] & m);
+            od = opaque((c.q[P][R >> 2][dw] >> 8) & m);
         } else {
-            // 6-bit codes per byte: ql nibble | 2 qh bits of quarter kh + 2(R>>2) at bits 4, 5
-            const uint32_t l = c.ql[P][piece][dw], h = c.qh[P][piece][dw];
-            const uint32_t u = R < 4 ? (l & 0x0f0f0f0fu) | ((h << (4u - 2u * kh)) & 0x30303030u)
-                                     : ((l >> 4) & 0x0f0f0f0fu) | ((h >> (2u * kh)) & 0x30303030u);
+            // 6-bit codes per byte: ql nibble | 2 qh bits (at 2q) of quarter q at bits 4, 5
+            constexpr int q = R >> 1;
+            const uint32_t l = c.ql[P][q & 1][dw], h = c.qh[P][dw];
+            const uint32_t u = ((q < 2 ? l : l >> 4) & 0x0f0f0f0fu) |
+                               ((q < 2 ? h << (4 - 2 * q) : h >> (2 * q - 4)) & 0x30303030u);
             ev = opaque(u & 0x00ff00ffu);
             od = opaque((u >> 8) & 0x00ff00ffu);
         }
@@ -255,15 +256,13 @@ __device__ __forceinline__ half8 mm_dequant(const MmCodes<FMT>& c, uint32_t kh, 
 
 // 16-byte piece (8 elements) of a 128-column stage row that half-wave kh
 // multiplies in step r: mm_piece0(kh) ^ mm_piece_step(r) (their bits are apart).
-template <int FMT>
 __device__ __forceinline__ constexpr uint32_t mm_piece0(uint32_t kh)
 {
-    return kh * (FMT == kFmtQ4 ? 8u : 4u);
+    return kh * 2u;
 }
-template <int FMT>
 __device__ __forceinline__ constexpr uint32_t mm_piece_step(int r)
 {
-    return FMT == kFmtQ4 ? uint32_t(r) : uint32_t(r >> 2) * 8u + uint32_t(r & 3);
+    return uint32_t(r >> 1) * 4u + uint32_t(r & 1);
 }
 
 // v / (1 + e^-v) for an fp16 result: one v_exp_f32 and one v_rcp_f32 (each
@@ -319,7 +318,7 @@ struct Mm {
         wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         kh = lane >> 5;
         const uint32_t wm = wave / WN;
-        frag = (wm * MF * 32u + l31) * kMmRowB + ((mm_piece0<FMT>(kh) ^ (l31 & 15u)) << 4);
+        frag = (wm * MF * 32u + l31) * kMmRowB + ((mm_piece0(kh) ^ (l31 & 15u)) << 4);
         xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(p.x), (short)0, int(p.M * p.ldx * 2u), 0x00020000);
         // fill i of this wave: stage rows 4*(wave*kFill + i) + lane/16; the lane's
         // 16 bytes land at piece lane%16 of that row, which holds source piece
@@ -355,13 +354,13 @@ struct Mm {
     // X fragment i of step r.
     __device__ __forceinline__ half8 frag_at(const uint8_t* stage, int r, int i) const
     {
-        return *reinterpret_cast<const half8*>(stage + (frag ^ (mm_piece_step<FMT>(r) << 4)) + i * (32 * kMmRowB));
+        return *reinterpret_cast<const half8*>(stage + (frag ^ (mm_piece_step(r) << 4)) + i * (32 * kMmRowB));
     }
 
     // Half P of super-block kb's codes, and with half 0 its scales: kLoads<P>
     // load instructions.
     template <int P>
-    static constexpr int kLoads = NF * (FMT == kFmtQ4 ? 2 + (P == 0) : 4 + 2 * (P == 0));
+    static constexpr int kLoads = NF * (FMT == kFmtQ4 ? 2 + (P == 0) : 3 + 2 * (P == 0));
     template <int P>
     __device__ __forceinline__ void load_w(uint32_t kb, MmCodes<FMT> (&c)[NF])
     {
@@ -379,8 +378,8 @@ struct Mm {
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             if constexpr (P == 0 && R == 0) mm_unpack<FMT>(hdr[f], kh, scale[f]);
-            if constexpr (R % mm_factor_steps<FMT>() == 0) mm_factors<FMT, P, R>(scale[f], fa[f], fn[f]);
-            o[f] = mm_dequant<FMT, P, R>(codes[f], kh, fa[f], fn[f]);
+            if constexpr (R % kMmFactorSteps == 0) mm_factors<FMT, P, R>(scale[f], fa[f], fn[f]);
+            o[f] = mm_dequant<FMT, P, R>(codes[f], fa[f], fn[f]);
         }
     }
 
