@@ -265,14 +265,14 @@ __device__ __forceinline__ constexpr uint32_t mm_piece_step(int r)
     return uint32_t(r >> 1) * 4u + uint32_t(r & 1);
 }
 
-// v / (1 + e^-v) for an fp16 result: one v_exp_f32 and one v_rcp_f32 (each
-// within an ulp of fp32) instead of the library's expf and an IEEE division,
-// some 20 instructions less per value: gate/up at 256 rows 79.4 -> 75.8 us; the
-// error of the fp16 result against float64 is its rounding's as before (3.6e-4).
-// +-inf and NaN as the quotient has them.
+// v / (1 + e^-v) with the library's exponential and an IEEE division: within 1.7e-7
+// of the exact value.  v_exp_f32(v * -log2 e) and v_rcp_f32 take some 20
+// instructions less per value (gate/up at 256 rows 74.9 against 77.6 us, at 100
+// rows 40.9 against 42.8), but the product's rounding enters the exponent, so
+// the relative error grows with |v| (1.0e-6 at |v| = 20) and fp16 results flip.
 __device__ __forceinline__ float mm_silu(float v)
 {
-    return v * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v * -1.44269504f));
+    return v / (1.0f + expf(-v));
 }
 
 // Workgroup barrier ordering LDS only: global loads in flight stay in flight.

@@ -2,8 +2,8 @@
 rounding of one product, sum or exponential into 5e-3 of its logits, far more
 than the bounds of the parity tests see in a single kernel, so each kernel's
 output is pinned by a SHA-256 recorded on an MI355X from the first MFMA kernels
-of the pass (commit 7d20864): the order in which products are summed and the
-rounding of decoded weights.  Whoever changes one of these on purpose measures
+of the pass (commit 7d20864): the order in which products are summed, the rounding
+of decoded weights and the SiLU.  Whoever changes one of these on purpose measures
 its error against float64 and records the digests again."""
 import hashlib
 
@@ -52,6 +52,13 @@ def qkv(v, H, kvd, K, M):
     return digest(y.download(np.uint32))
 
 
+def gateup(N, K, M):
+    s, ws = arc.DeviceBuffer(M * N * 2), arc.DeviceBuffer(arc.prefill_gemm_workspace_bytes(N, K))
+    # gate values of some tens on both sides of zero, products inside fp16's range
+    arc.prefill_gateup(weights(arc.Q4_K, N, K, 7), weights(arc.Q4_K, N, K, 8), N, K, rows16(M, K, 9, 0.3), M, s, ws)
+    return digest(s.download(np.uint16))
+
+
 # 2560 x 10240: 10 splits of 4 super-blocks
 PINNED = [
     (gemm, (arc.Q4_K, 200, 1536, 70), "65a222e9a52fcd9d"),
@@ -60,6 +67,8 @@ PINNED = [
     (gemm, (arc.Q6_K_PADDED, 2560, 10240, 100), "361d44d227dc8647"),
     (qkv, (arc.Q4_K, 512, 256, 512, 23), "b64906c7b95aeb00"),
     (qkv, (arc.Q6_K_PADDED, 512, 256, 1024, 150), "7fa4f3692e91c8f8"),
+    (gateup, (200, 1024, 100), "bc1cdfbaf041a142"),
+    (gateup, (2048, 512, 256), "f39bd34dfea392e2"),
 ]
 
 
