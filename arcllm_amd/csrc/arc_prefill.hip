@@ -336,13 +336,14 @@ __global__ __launch_bounds__(256) void k_pf_attn(const float* __restrict__ q, co
 //  softmax the chunk maximum of a query from the lane's 32 scores and its
 //          partner half-wave's (lane ^ 32); positions past the query's own
 //          are masked.  Weights e^(x - max), rescaling the running sum and
-//          the output by e^(max_old - max_new), as powers of two of scores
-//          times log2(e).
+//          the output by e^(max_old - max_new).
 //  Bound by vector instructions: one wave per SIMD, 64 weights per lane and
-//  chunk.  256 rows at position 768, 28 heads: 20.1 us, 24.8 with expf (about 10
-//  instructions each against one v_exp_f32) and the mask compared in every
-//  chunk; 8 waves per workgroup (half the chunks each) 26.0; the weights' hi and
-//  lo parts by v_cvt_pk_f16_f32 and skipping rescalings by 1 changed nothing.
+//  chunk, about 10 instructions each for expf.  256 rows at position 768, 28
+//  heads: 21.7 us, 24.8 with the mask compared in every chunk; 8 waves per
+//  workgroup (half the chunks each) 26.0; the weights' hi and lo parts by
+//  v_cvt_pk_f16_f32 and skipping rescalings by 1 changed nothing.  Weights as
+//  v_exp_f32 of scores times log2(e) take 20.1 us and are as accurate, but round
+//  differently, and a prompt's logits move by 5e-3 with them.
 //  values  O^T = V^T P^T: B = P^T straight from the lane's weights (step s of
 //          a tile: values 8s .. 8s+7, keys 16s + 8(j/4) + 4(lane/32) + j%4)
 //          as fp16 hi + lo; A = V^T from LDS, where the wave stages its chunk
@@ -371,7 +372,6 @@ __global__ __launch_bounds__(256, 2) void k_pf_attn_mf(const float* __restrict__
     const uint32_t q0 = b * 32, qlast = min(q0 + 31, M - 1);
     const uint32_t qpos = pos0 + q0 + uint32_t(l32);  // this lane's query position
     const uint32_t nkc = (pos0 + qlast + kChunk) / kChunk;  // chunks holding positions 0 .. pos0 + qlast
-    const float scale2 = scale * 1.44269504f;               // weights e^x as 2^(x log2 e), one v_exp_f32 each
 
     half8 qh[8], ql[8];  // B operand of the scores: query l32, dims 16s + 8 h2 .. +7
     {
@@ -439,15 +439,15 @@ __global__ __launch_bounds__(256, 2) void k_pf_attn_mf(const float* __restrict__
                 for (int j = 0; j < 8; ++j) vw[8 * e + j][col] = v8[j];
             }
         }
-        // scores times scale * log2(e), masked in the chunks that reach past the
-        // block's first query; the chunk maximum per query
+        // scaled scores, masked in the chunks that reach past the block's first
+        // query; the chunk maximum per query
         float mx = -INFINITY;
         if (kbase + kChunk - 1 <= pos0 + q0) {
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    sc[kt][i] *= scale2;
+                    sc[kt][i] *= scale;
                     mx = fmaxf(mx, sc[kt][i]);
                 }
         } else {
@@ -456,7 +456,7 @@ __global__ __launch_bounds__(256, 2) void k_pf_attn_mf(const float* __restrict__
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const uint32_t kpos = kbase + 32u * kt + 8u * (i >> 2) + 4u * h2 + (i & 3);
-                    const float v = kpos <= qpos ? sc[kt][i] * scale2 : -INFINITY;
+                    const float v = kpos <= qpos ? sc[kt][i] * scale : -INFINITY;
                     sc[kt][i] = v;
                     mx = fmaxf(mx, v);
                 }
@@ -464,13 +464,13 @@ __global__ __launch_bounds__(256, 2) void k_pf_attn_mf(const float* __restrict__
         mx = xor_max<32>(mx);
         const float mnew = fmaxf(mrun, mx);
         const float mr = mnew == -INFINITY ? 0.0f : mnew;  // no position <= the query's yet: all weights 0
-        const float alpha = __builtin_amdgcn_exp2f(mrun - mr);  // mrun = -inf: 0
+        const float alpha = expf(mrun - mr);              // mrun = -inf: 0
         float es = 0.0f;
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const float e = __builtin_amdgcn_exp2f(sc[kt][i] - mr);
+                const float e = expf(sc[kt][i] - mr);
                 sc[kt][i] = e;
                 es += e;
             }
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(256, 2) void k_pf_attn_mf(const float* __restrict__
     float f[4], L = 0.0f;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        f[v] = __builtin_amdgcn_exp2f(mw[v][qq] - Mx);
+        f[v] = expf(mw[v][qq] - Mx);
         L = __builtin_fmaf(lw[v][qq], f[v], L);
     }
     const float li = 1.0f / L;

@@ -1,16 +1,18 @@
 """The prompt pass's results bit for bit.  A prompt's 28 layers turn a changed
 rounding of one product, sum or exponential into 5e-3 of its logits, far more
 than the bounds of the parity tests see in a single kernel, so each kernel's
-output is pinned by a SHA-256 recorded on an MI355X from the first MFMA kernels
-of the pass (commit 7d20864): the order in which products are summed, the rounding
-of decoded weights and the SiLU.  Whoever changes one of these on purpose measures
-its error against float64 and records the digests again."""
+output (and a small model's logits and caches) is pinned by a SHA-256 recorded
+on an MI355X from the first MFMA kernels of the pass (commit 7d20864): the order
+in which products are summed, the rounding of decoded weights, the SiLU and the
+softmax.  Whoever changes one of these on purpose measures its error against
+float64 and records the digests again."""
 import hashlib
 
 import numpy as np
 import pytest
 
 import arcllm_amd as arc
+from decode_common import tiny_dims
 
 pytestmark = pytest.mark.gpu
 
@@ -59,6 +61,28 @@ def gateup(N, K, M):
     return digest(s.download(np.uint16))
 
 
+def attention(kv_heads, hpk, pos0, M, mfma):
+    ctx, n = pos0 + M, kv_heads * hpk * 128
+    kc, vc = rows16(ctx, kv_heads * 128, 10), rows16(ctx, kv_heads * 128, 11)
+    x = arc.DeviceBuffer(M * n * 2)
+    arc.prefill_attention(dev(arc.synth_normal(SEED, 12, M * n) * np.float32(2.0)), kc, vc, kv_heads, hpk, ctx, pos0, M, x,
+                          n, mfma=mfma)
+    return digest(x.download(np.uint16))
+
+
+def prompt(layers, n):
+    d = tiny_dims(layers)
+    s = arc.Session(arc.Model(d, seed=SEED), n)
+    s.prefill((np.arange(n, dtype=np.uint32) * 61 + 5) % d.vocab, logits=True)
+    got = [s.logits()]
+    for layer in range(layers):
+        for p in s.kv(layer):
+            h = np.empty(n * d.kv_heads * 128, np.uint16)
+            arc.check(arc.lib().arc_memcpy_dtoh(h.ctypes.data, p, h.nbytes, None))
+            got.append(h)
+    return digest(*got)
+
+
 # 2560 x 10240: 10 splits of 4 super-blocks
 PINNED = [
     (gemm, (arc.Q4_K, 200, 1536, 70), "65a222e9a52fcd9d"),
@@ -69,6 +93,10 @@ PINNED = [
     (qkv, (arc.Q6_K_PADDED, 512, 256, 1024, 150), "7fa4f3692e91c8f8"),
     (gateup, (200, 1024, 100), "bc1cdfbaf041a142"),
     (gateup, (2048, 512, 256), "f39bd34dfea392e2"),
+    (attention, (2, 7, 300, 70, True), "a2fb4329a706cae2"),
+    (attention, (3, 2, 0, 256, True), "e52f36b1b0bf8257"),
+    (attention, (2, 7, 300, 70, False), "c5b278c8ae9a2993"),
+    (prompt, (3, 300), "15d5ab12a2e64d46"),
 ]
 
 
