@@ -827,8 +827,8 @@ struct PfWorkspace {
     size_t x, part, bytes;
 };
 
-// X staging (256 rows of K fp16, for rows at odd addresses) and the split
-// partials of the N x K projection's plan.
+// X staging (256 rows of K fp16, see pf_stage_x) and the split partials of the N
+// x K projection's plan.
 PfWorkspace pf_workspace(uint32_t N, uint32_t K)
 {
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -852,15 +852,20 @@ int pf_check(const void* w, uint32_t N, uint32_t K, const uint16_t* x, uint32_t 
     return ARC_OK;
 }
 
-// The GEMM's X: the given rows, or, where they do not start at a 16-byte
-// boundary (the tiles read 16 bytes at a time), a copy of them in the workspace.
-int pf_stage_x(uint8_t* ws, const PfWorkspace& w, const uint16_t* x, uint32_t M, uint32_t K, hipStream_t st, PfGemm& g)
+// The GEMM's X: the given rows, or a copy of them in the workspace where they do
+// not start at a 16-byte boundary (the tiles read 16 bytes at a time) or share
+// memory with the `out_bytes` at `out` that the GEMM launch writes (a workgroup
+// that has finished stores while others still read X).
+int pf_stage_x(uint8_t* ws, const PfWorkspace& w, const uint16_t* x, uint32_t M, uint32_t K, const void* out, size_t out_bytes,
+               hipStream_t st, PfGemm& g)
 {
+    const size_t bytes = size_t(M) * K * sizeof(_Float16);
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), oa = reinterpret_cast<uintptr_t>(out);
     g.ldx = K;
     g.x = reinterpret_cast<const _Float16*>(x);
-    if ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) return ARC_OK;
+    if ((xa & 15u) == 0 && (xa + bytes <= oa || oa + out_bytes <= xa)) return ARC_OK;
     g.x = reinterpret_cast<const _Float16*>(ws + w.x);
-    return check_hip(hipMemcpyAsync(ws + w.x, x, size_t(M) * K * sizeof(_Float16), hipMemcpyDeviceToDevice, st), "x staging");
+    return check_hip(hipMemcpyAsync(ws + w.x, x, bytes, hipMemcpyDeviceToDevice, st), "x staging");
 }
 
 // y[m][c] = sum over the splits of part[s][m][c], in split order.
@@ -902,7 +907,7 @@ int arc_prefill_gemm(int qtype, const void* w, uint32_t N, uint32_t K, const uin
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     const PfWorkspace pw = pf_workspace(N, K);
     PfGemm g{};
-    if ((rc = pf_stage_x(ws, pw, x, M, K, st, g))) return rc;
+    if ((rc = pf_stage_x(ws, pw, x, M, K, ws + pw.part, pw.bytes - pw.part, st, g))) return rc;
     g.M = M;
     g.mpad = kPfMaxM;
     g.nb = K / kQK;
@@ -928,7 +933,7 @@ int arc_prefill_gateup(const void* w_gate, const void* w_up, uint32_t N, uint32_
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     const PfWorkspace pw = pf_workspace(N, K);
     PfGemm u{};
-    if ((rc = pf_stage_x(ws, pw, x, M, K, st, u))) return rc;
+    if ((rc = pf_stage_x(ws, pw, x, M, K, s, size_t(M) * N * sizeof(_Float16), st, u))) return rc;
     u.M = M;
     u.mpad = kPfMaxM;
     u.nb = K / kQK;
@@ -988,7 +993,7 @@ int arc_prefill_qkv(const void* wq, const void* wk, const void* wv, int v_qtype,
     const PfWorkspace pw = pf_workspace(N, K);
     // as run_prefill: partials [split][mpad][H | kvd | kvd]
     PfGemm g{};
-    if ((rc = pf_stage_x(ws, pw, x, M, K, st, g))) return rc;
+    if ((rc = pf_stage_x(ws, pw, x, M, K, ws + pw.part, pw.bytes - pw.part, st, g))) return rc;
     g.M = M;
     g.mpad = kPfMaxM;
     g.nb = K / kQK;

@@ -215,7 +215,9 @@ int arc_attention_decode(const float *q, const void *kc, const void *vc, uint32_
                          uint32_t max_ctx, uint32_t T, float *out, void *workspace, arc_stream_t stream);
 
 /* Bytes of device workspace the prompt-pass projection entry points need for
- * an N x K weight (fp16 X staging of 256 rows and the split-K partials). */
+ * an N x K weight: room for 256 fp16 rows of X, which are copied there where x is
+ * not 16-byte aligned or shares memory with what the product writes, and the
+ * split-K partials. */
 size_t arc_prefill_gemm_workspace_bytes(uint32_t N, uint32_t K);
 
 /* The prompt pass's projection GEMM, with its kernel and split-K plan:
@@ -229,7 +231,7 @@ int arc_prefill_gemm(int qtype, const void *w, uint32_t N, uint32_t K, const uin
 
 /* The prompt pass's fused gate/up + SwiGLU GEMM (Q4_K gate and up):
  * s[m][n] = fp16(silu(g) * u), g = x w_gate^T, u = x w_up^T, for m < M <= 256.
- * x: fp16 bits [M][K]; s: fp16 bits [M][N].  workspace as for
+ * x: fp16 bits [M][K]; s: fp16 bits [M][N], may overlap x.  workspace as for
  * arc_prefill_gemm.  Replaces p7l (src/arcllm_v1_runtime.cpp:340-369). */
 int arc_prefill_gateup(const void *w_gate, const void *w_up, uint32_t N, uint32_t K, const uint16_t *x, uint32_t M,
                        uint16_t *s, void *workspace, arc_stream_t stream);
