@@ -125,7 +125,7 @@ __device__ __forceinline__ u32x4 mm_ld16(__amdgpu_buffer_rsrc_t w, uint32_t voff
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w, voff, soff, 0));
 }
 
-// Through a buffer descriptor over the tile's weight rows: `row` is the
+// Through a buffer descriptor over the wave's weight rows: `row` is the
 // lane's row, `blk` (uniform) the super-block's offset in it.
 template <int FMT, int P>
 __device__ __forceinline__ void mm_load_codes(__amdgpu_buffer_rsrc_t w, uint32_t row, uint32_t blk, uint32_t kh,
@@ -309,7 +309,7 @@ struct Mm {
     uint32_t frag;              // byte address of step 0's piece of the lane's first row
     uint32_t voff[kFill];       // byte offsets of the lane's fills (column 0)
     __amdgpu_buffer_rsrc_t xr;
-    __amdgpu_buffer_rsrc_t wr;  // the tile's weight rows
+    __amdgpu_buffer_rsrc_t wr;  // the wave's weight rows
     uint32_t wrow[NF];          // byte offsets of the lane's rows
 
     __device__ __forceinline__ void init_x(const PfGemm& p)
@@ -480,11 +480,14 @@ __device__ __forceinline__ void mm_body(const PfGemm& p, uint32_t tile, uint8_t*
     const bool up = SWIGLU && wn >= WN / 2;
     const uint32_t c0 = (SWIGLU ? wn % (WN / 2) : wn) * (NF * 32u);  // the wave's first column in the tile
     const uint32_t kb0 = SWIGLU ? 0u : blockIdx.y * p.bps, kb1 = SWIGLU ? p.nb : min(p.nb, kb0 + p.bps);
-    const uint32_t row0 = tile * kCols, rows = min(p.N - row0, uint32_t(kCols));  // row0 < N
-    t.wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(up ? p.w1 : p.w0) + uint64_t(row0) * p.row_bytes, (short)0,
+    const uint32_t row0 = tile * kCols;  // < N
+    // the wave's own weight rows (past N: the last row again), so that 32-bit
+    // offsets reach every K that the host lets through
+    const uint32_t first = min(row0 + c0, p.N - 1u), rows = min(p.N - first, NF * 32u);
+    t.wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(up ? p.w1 : p.w0) + uint64_t(first) * p.row_bytes, (short)0,
                                              int(rows * uint32_t(p.row_bytes)), 0x00020000);
 #pragma unroll
-    for (int f = 0; f < NF; ++f) t.wrow[f] = min(c0 + f * 32u + l31, rows - 1u) * uint32_t(p.row_bytes);
+    for (int f = 0; f < NF; ++f) t.wrow[f] = min(f * 32u + l31, rows - 1u) * uint32_t(p.row_bytes);
     t.run(s0, s1, kb0, kb1);
 
     auto quad = [&](int f, int i, int q) {

@@ -846,6 +846,10 @@ int pf_check(const void* w, uint32_t N, uint32_t K, const uint16_t* x, uint32_t 
         return set_error(ARC_ERR_INVALID_ARGUMENT, "bad shape N=%u K=%u M=%u (K a multiple of 256, 1 <= M <= %d)", N, K,
                          M, kPfMaxM);
     if (N > uint32_t(kResCols) * 1024u) return set_error(ARC_ERR_UNSUPPORTED, "N must be <= %d", kResCols * 1024);
+    // the tiles' 32-bit offsets: M rows of X (2 M K bytes) and 32 weight rows (212
+    // bytes for 256 columns at most)
+    if (uint64_t(M) * K >= (uint64_t(1) << 31) || K > (1u << 27))
+        return set_error(ARC_ERR_UNSUPPORTED, "K=%u: M * K must be below 2^31 and K at most 2^27", K);
     if (reinterpret_cast<uintptr_t>(w) & 15u) return set_error(ARC_ERR_INVALID_ARGUMENT, "weights not 16-byte aligned");
     if (reinterpret_cast<uintptr_t>(ws) & 255u)
         return set_error(ARC_ERR_INVALID_ARGUMENT, "workspace must be 256-byte aligned");

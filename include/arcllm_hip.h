@@ -223,8 +223,8 @@ size_t arc_prefill_gemm_workspace_bytes(uint32_t N, uint32_t K);
 /* The prompt pass's projection GEMM, with its kernel and split-K plan:
  * y[m][n] = sum_k x[m][k] w[n][k] for m < M <= 256, fp16 operands (each
  * weight decoded in fp32 and rounded to fp16), fp32 accumulation, the split
- * partials added in split order.  x: fp16 bits [M][K]; w: [N x K] Q4_K or
- * ARC_Q6_K_PADDED; y: fp32 [M][N].  Replaces the p7c/p7g tiled GEMM
+ * partials added in split order.  x: fp16 bits [M][K], M * K < 2^31, K <= 2^27;
+ * w: [N x K] Q4_K or ARC_Q6_K_PADDED; y: fp32 [M][N].  Replaces the p7c/p7g tiled GEMM
  * dispatches of build_prefill (src/arcllm_v1_runtime.cpp:340-369). */
 int arc_prefill_gemm(int qtype, const void *w, uint32_t N, uint32_t K, const uint16_t *x, uint32_t M, float *y,
                      void *workspace, arc_stream_t stream);
