@@ -485,29 +485,41 @@ static void launch_attn_w(const AttnParams& ap, uint32_t nsplit, uint32_t kv_hea
     }
 }
 
+// Whether a call at a known context T > 0 takes 8 waves per workgroup (past 4096
+// positions, where 4 waves take two chunks per split, two 8-wave chunks) instead
+// of 4.  For it: the merge reads every split's partials in one workgroup per kv
+// head, and 8 waves halve the splits.  Against it: an 8-wave workgroup has a CU to
+// itself (145 registers are three waves per SIMD, and it takes two), so more than
+// 256 of them run in two rounds, and fewer than 96 leave the loads to too few CUs
+// where a split has two chunks.  us per call, 4 waves / 8 waves
+// (kv heads x query heads per kv head; [workgroups of 8 waves]):
+//   T = 2049   1x1  9.1 /  9.5   3x3 10.3 / 10.6   4x7 12.9 / 12.5   8x8 14.8 / 13.3  24x2 18.4 / 17.1  32x8 26.6 / 28.6
+//   T = 2600   1x1  9.6 /  9.8   2x8 13.1 / 12.8   4x8 13.9 / 13.1   8x8 17.6 / 14.1  16x8 24.3 / 21.4  32x8 28.2 / 29.9
+//   T = 3100   1x1 10.2 /  9.9   2x8 14.0 / 13.0   4x8 15.3 / 13.5   8x8 19.5 / 14.5  16x8 27.3 / 22.6  32x8 36.1 / 35.3
+//   T = 4096   1x1 10.7 / 10.2   2x7 14.6 / 12.9   4x7 16.3 / 13.6   8x8 21.9 / 15.5  16x8 30.6 / 24.9  64x8 70.8 / 76.4
+//   T = 4097   4x7 [68] 14.8 / 15.5   5x3 [85] 12.6 / 13.1   6x4 [102] 13.6 / 13.4   8x8 [136] 18.2 / 16.4
+//   T = 5120   4x7 [80] 15.5 / 15.6   5x3 [100] 13.3 / 13.2  12x4 [240] 18.0 / 14.7  15x2 [300] 19.1 / 21.3
+//   T = 8192   4x7 [128] 18.1 / 16.2  7x8 [224] 22.7 / 17.6   8x3 [256] 19.1 / 14.8   9x4 [288] 21.8 / 25.2
+//   T = 8193   4x7 [132] 17.5 / 17.2  7x8 [231] 22.0 / 18.8   8x3 [264] 17.1 / 19.0  10x8 [330] 22.9 / 28.3
+//   T = 32768  4x7 [256] 27.2 / 25.6  5x7 [320] 34.6 / 38.6   8x8 [512] 36.8 / 44.5
+static bool attn_eight_waves(uint32_t T, uint32_t kv_heads)
+{
+    if (T <= 2048) return false;
+    if (T <= 4096) return kv_heads >= 4 && kv_heads <= 24 ? true : T > 3072 && kv_heads <= 32;
+    const uint32_t wgs = attn_split(T, 8 * kAttnTile, 2).nsplit * kv_heads;
+    return kv_heads >= 4 && wgs >= 96 && wgs <= 256;
+}
+
 // Sets ap.min_cps and launches.  T = 0: the position is only known on the
 // device (grid kMaxSplits x kv heads; workgroups past its plan return at once).
-// Otherwise the grid is the plan's, and the shape follows the context: the
-// merge reads every split's partials in one workgroup per kv head, so past 2048
-// positions half as many splits of 8 waves win, and past 4096, where 4 waves
-// take two chunks per split, two 8-wave chunks do for 4 kv heads or more (us per
-// call, 4 waves / 8 waves; kv heads x query heads per kv head):
-//   T = 2000  4x7 12.0 / 11.9   1x8 11.5 / 11.9   8x4 13.1 / 11.3   2x2  9.2 /  9.8
-//   T = 2500  4x7 13.6 / 12.8   1x8 12.7 / 12.6   8x4 14.7 / 12.1   2x2 10.1 / 10.0
-//   T = 4001  4x7 16.2 / 13.7   1x8 14.2 / 13.2   8x4 18.5 / 13.6   2x2 11.7 / 10.6
-//   T = 6000  4x7 16.6 / 15.9   1x8 15.0 / 16.1   8x4 17.2 / 14.5   2x2 11.9 / 12.6
-//   T = 8192  4x7 18.0 / 16.1   1x8 16.3 / 16.6   8x4 19.9 / 15.2   2x2 13.3 / 13.0
+// Otherwise the grid is the plan's, and attn_eight_waves picks the shape.
 static void launch_attn(AttnParams ap, uint32_t kv_heads, hipStream_t st, uint32_t T = 0)
 {
     int waves = g_attn_waves ? g_attn_waves : 4;
     ap.min_cps = g_attn_min_cps > 0 ? uint32_t(g_attn_min_cps) : 1u;
-    if (!g_attn_waves && g_attn_min_cps <= 0) {
-        if (T > 4096 && kv_heads >= 4) {
-            waves = 8;
-            ap.min_cps = 2;
-        } else if (T > 2048 && T <= 4096) {
-            waves = 8;
-        }
+    if (!g_attn_waves && g_attn_min_cps <= 0 && attn_eight_waves(T, kv_heads)) {
+        waves = 8;
+        ap.min_cps = T > 4096 ? 2u : 1u;
     }
     const uint32_t nsplit = T ? attn_split(T, uint32_t(waves) * kAttnTile, ap.min_cps).nsplit : uint32_t(kMaxSplits);
     if (waves == 8)

@@ -201,8 +201,11 @@ int arc_lmhead_argmax_noalloc(int qtype, const void *w, uint32_t rows, uint32_t 
  * arrival counters, control block); 0 for unsupported head counts. */
 size_t arc_attention_workspace_bytes(uint32_t kv_heads, uint32_t hpk);
 
-/* Cached GQA attention of one decode position, with the decode step's kernel
- * and split plan: out[h*128 + d] = sum_t softmax_t(q_h . k_t / sqrt(128))
+/* Cached GQA attention of one decode position, with the decode step's kernel.
+ * Up to 2048 positions its splits are the decode step's too; past that the call,
+ * which knows T on the host, picks waves and splits by T and kv_heads (a captured
+ * step takes 4 waves at every position), and sums in that order:
+ * out[h*128 + d] = sum_t softmax_t(q_h . k_t / sqrt(128))
  * v_t[d] over positions t < T, query head h reading kv head h / hpk.
  * q, out: fp32 [kv_heads*hpk*128] (16-byte aligned); kc, vc: fp16
  * [max_ctx][kv_heads*128] (16-byte aligned); 1 <= T <= max_ctx <= 32768;

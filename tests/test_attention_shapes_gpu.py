@@ -38,3 +38,40 @@ def test_shape_by_context(kv_heads, hpk, T):
     ref = orc.attention_decode_f64(q, kc, vc, T, kv_heads * hpk, kv_heads)
     assert orc.rel_err(got[0], ref) <= 1e-3
     assert np.max(np.abs(got[0] - got[1])) <= 3.6e-4 * np.max(np.abs(ref))
+
+
+# (kv heads, query heads per kv head, T) and the shape the rule gives: both sides
+# of each of its lines (2048, 3072, 4096 positions; 4, 24 and 32 kv heads; 96 and
+# 256 workgroups of 8 waves)
+LINES = [
+    (4, 7, 2048, (4, 1)), (4, 7, 2049, (8, 1)), (24, 1, 2049, (8, 1)), (25, 1, 3072, (4, 1)), (25, 1, 3073, (8, 1)),
+    (33, 1, 3073, (4, 1)), (3, 8, 3072, (4, 1)), (3, 8, 3073, (8, 1)), (8, 8, 4096, (8, 1)), (2, 7, 4097, (4, 1)),
+    (4, 7, 4097, (4, 1)), (4, 7, 5888, (4, 1)), (4, 7, 5889, (8, 2)), (6, 8, 4097, (8, 2)), (8, 4, 8192, (8, 2)),
+    (8, 4, 8193, (4, 1)), (12, 2, 5376, (8, 2)), (12, 2, 5377, (4, 1)), (7, 8, 9216, (8, 2)), (7, 8, 9217, (4, 1)),
+    (4, 2, 32768, (8, 2)), (5, 2, 32768, (4, 1)),
+]
+
+
+@pytest.mark.parametrize("kv_heads,hpk,T,shape", LINES, ids=["%dx%d-%d" % c[:3] for c in LINES])
+def test_rule(kv_heads, hpk, T, shape):
+    """The automatic call gives the bits of the shape that the rule names (another
+    shape adds in another order and differs in some), and is right."""
+    n = kv_heads * hpk * 128
+    kc = arc.synth_normal(SEED, 11, T * kv_heads * 128).astype(np.float16)
+    vc = arc.synth_normal(SEED, 12, T * kv_heads * 128).astype(np.float16)
+    q = arc.synth_normal(SEED, 13 + T, n) * np.float32(2.0)
+    dk, dv, dq = dev(kc), dev(vc), dev(q)
+    ws = arc.DeviceBuffer(arc.attention_workspace_bytes(kv_heads, hpk))
+    got = {}
+    for tune in ((0, 0), (4, 1), (8, 2 if T > 4096 else 1)):
+        out = arc.DeviceBuffer(n * 4)
+        arc.tune_attention(*tune)
+        try:
+            arc.attention_decode(dq, dk, dv, kv_heads, hpk, T, T, out, ws)
+        finally:
+            arc.tune_attention()
+        got[tune] = out.download(np.uint32)
+    for tune in list(got)[1:]:
+        assert np.array_equal(got[0, 0], got[tune]) == (tune == shape), tune
+    ref = orc.attention_decode_f64(q, kc, vc, T, kv_heads * hpk, kv_heads)
+    assert orc.rel_err(got[0, 0].view(np.float32), ref) <= 1e-3
