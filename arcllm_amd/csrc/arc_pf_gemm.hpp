@@ -2,8 +2,8 @@
 // MFMA): Y[m][n] = sum_k X[m][k] W[n][k], X fp16, W Q4_K or padded Q6_K
 // decoded to fp16 in registers, fp32 accumulation.
 //
-// Workgroup of WM x WN waves, wave (wm, wn) owns MF*32 rows of X and NF*32
-// weight rows with v_mfma_f32_32x32x16_f16 (lane l: X row / weight row l%32,
+// Workgroup of WN waves; each takes all MF*32 rows of X in the tile and 32 weight
+// rows of its own with v_mfma_f32_32x32x16_f16 (lane l: X row / weight row l%32,
 // 8 of the 16 K elements by half-wave kh = l/32).  The K order is the one that
 // every kernel of the prompt pass has summed in (half block p of 128 elements,
 // step r of 8, half-wave kh):
@@ -25,7 +25,7 @@
 // and two of their eight issue slots, so six other vector instructions are free
 // with two waves per SIMD (a 16x16x32 one takes 16 cycles and leaves two); the
 // decode costs 2.25 per weight (0.75 to mask the codes, v_fma_mix_f32, half a
-// v_cvt_pk_f16_f32).  Each wave takes all rows of the pass (WM = 1), so a weight
+// v_cvt_pk_f16_f32).  Each wave takes all rows of the pass, so a weight
 // is decoded once and feeds up to 8 MFMAs: 2.4 other vector instructions and
 // one LDS read (4 cycles of the LDS) per MFMA.  Gate/up 18944 x 3584 at 256 rows
 // (whole call): 76 us, 917 TFLOP/s, 100 us before (34 instructions to decode 8
@@ -285,40 +285,39 @@ __device__ __forceinline__ void lds_barrier()
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-template <int FMT, int MF, int NF, int WM, int WN>
+template <int FMT, int MF, int WN>
 struct Mm {
-    static constexpr int W = WM * WN;
-    static constexpr int kRows = 32 * MF * WM;           // X rows of the tile
+    static constexpr int kRows = 32 * MF;                // X rows of the tile
     static constexpr int kStageB = kRows * kMmRowB;      // bytes of a stage
-    static constexpr int kFill = kRows / 4 / W;          // 1 KB fills (4 rows) per wave and stage
+    static constexpr int kFill = kRows / 4 / WN;          // 1 KB fills (4 rows) per wave and stage
     static constexpr int kD = 4;                         // X fragments held, read kD uses ahead
     static constexpr int kUses = 8 * MF;                 // X fragments of a stage
     static constexpr int kSync = kUses - kD / 2;         // fragment in front of which the stage changes
     static constexpr int kBB = mm_block_bytes<FMT>();
-    static_assert(kRows % (4 * W) == 0 && kUses % kD == 0, "whole fills per wave, whole rounds of the X ring");
+    static_assert(kRows % (4 * WN) == 0 && kUses % kD == 0, "whole fills per wave, whole rounds of the X ring");
 
-    f32x16 acc[NF][MF];
+    f32x16 acc[MF];
     half8 a[kD];
-    half8 b[2][NF];
-    MmCodes<FMT> codes[NF];     // in use
-    MmCodes<FMT> next[NF];      // in flight: 12 steps (about 3 us) from its load to its first use
-    MmHdr<FMT> hdr[NF];
-    MmScale<FMT> scale[NF];
-    float fa[NF], fn[NF];
+    half8 b[2];
+    MmCodes<FMT> codes;         // in use
+    MmCodes<FMT> next;          // in flight: 12 steps (about 3 us) from its load to its first use
+    MmHdr<FMT> hdr;
+    MmScale<FMT> scale;
+    float fa, fn;
     uint32_t kh, wave;
     uint32_t frag;              // byte address of step 0's piece of the lane's first row
     uint32_t voff[kFill];       // byte offsets of the lane's fills (column 0)
     __amdgpu_buffer_rsrc_t xr;
     __amdgpu_buffer_rsrc_t wr;  // the wave's weight rows
-    uint32_t wrow[NF];          // byte offsets of the lane's rows
+    uint32_t wrow;              // byte offset of the lane's row
 
     __device__ __forceinline__ void init_x(const PfGemm& p)
     {
         const uint32_t lane = threadIdx.x & 63u, l31 = lane & 31u;
         wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         kh = lane >> 5;
-        const uint32_t wm = wave / WN;
-        frag = (wm * MF * 32u + l31) * kMmRowB + ((mm_piece0(kh) ^ (l31 & 15u)) << 4);
+        // (opaque: seen through, the row offsets became ors instead of immediates)
+        frag = opaque(l31 * kMmRowB + ((mm_piece0(kh) ^ (l31 & 15u)) << 4));
         xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(p.x), (short)0, int(p.M * p.ldx * 2u), 0x00020000);
         // fill i of this wave: stage rows 4*(wave*kFill + i) + lane/16; the lane's
         // 16 bytes land at piece lane%16 of that row, which holds source piece
@@ -330,11 +329,9 @@ struct Mm {
             voff[i] = min(r, p.M - 1u) * p.ldx * 2u + (((lane & 15u) ^ (r & 15u)) << 4);
         }
 #pragma unroll
-        for (int f = 0; f < NF; ++f)
+        for (int i = 0; i < MF; ++i)
 #pragma unroll
-            for (int i = 0; i < MF; ++i)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) acc[f][i][j] = 0.0f;
+            for (int j = 0; j < 16; ++j) acc[i][j] = 0.0f;
     }
 
     // Part PART of 4 of this wave's share of columns [128 kx, 128 kx + 128) of X
@@ -360,27 +357,21 @@ struct Mm {
     // Half P of super-block kb's codes, and with half 0 its scales: kLoads<P>
     // load instructions.
     template <int P>
-    static constexpr int kLoads = NF * (FMT == kFmtQ4 ? 2 + (P == 0) : 3 + 2 * (P == 0));
+    static constexpr int kLoads = FMT == kFmtQ4 ? 2 + (P == 0) : 3 + 2 * (P == 0);
     template <int P>
-    __device__ __forceinline__ void load_w(uint32_t kb, MmCodes<FMT> (&c)[NF])
+    __device__ __forceinline__ void load_w(uint32_t kb, MmCodes<FMT>& c)
     {
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            if constexpr (P == 0) mm_load_hdr<FMT>(wr, wrow[f], kb * uint32_t(kBB), hdr[f]);
-            mm_load_codes<FMT, P>(wr, wrow[f], kb * uint32_t(kBB), kh, c[f]);
-        }
+        if constexpr (P == 0) mm_load_hdr<FMT>(wr, wrow, kb * uint32_t(kBB), hdr);
+        mm_load_codes<FMT, P>(wr, wrow, kb * uint32_t(kBB), kh, c);
     }
 
-    // Weight fragments of step (P, R).
+    // Weight fragment of step (P, R).
     template <int P, int R>
-    __device__ __forceinline__ void make_b(half8 (&o)[NF])
+    __device__ __forceinline__ half8 make_b()
     {
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            if constexpr (P == 0 && R == 0) mm_unpack<FMT>(hdr[f], kh, scale[f]);
-            if constexpr (R % kMmFactorSteps == 0) mm_factors<FMT, P, R>(scale[f], fa[f], fn[f]);
-            o[f] = mm_dequant<FMT, P, R>(codes[f], fa[f], fn[f]);
-        }
+        if constexpr (P == 0 && R == 0) mm_unpack<FMT>(hdr, kh, scale);
+        if constexpr (R % kMmFactorSteps == 0) mm_factors<FMT, P, R>(scale, fa, fn);
+        return mm_dequant<FMT, P, R>(codes, fa, fn);
     }
 
     // Step R of half P of super-block kb from stage `st`; kn is the next
@@ -395,15 +386,10 @@ struct Mm {
     __device__ __forceinline__ void step(uint8_t* st, uint8_t* ot, uint32_t kb, uint32_t kn)
     {
         constexpr int kNextP = R == 7 ? 1 - P : P, kNextR = (R + 1) & 7;
-        half8 (&bc)[NF] = b[R & 1];
-        half8 (&bn)[NF] = b[1 - (R & 1)];
         if constexpr (R < 3) fill<R + 1>(ot, (P == 0 ? kb : kn) * 2u + (1 - P));
         if constexpr (R == 3) load_w<P>(kn, next);
-        if constexpr (R == 7) {
-#pragma unroll
-            for (int f = 0; f < NF; ++f) mm_take<FMT, kNextP>(codes[f], next[f]);
-        }
-        make_b<kNextP, kNextR>(bn);
+        if constexpr (R == 7) mm_take<FMT, kNextP>(codes, next);
+        b[1 - (R & 1)] = make_b<kNextP, kNextR>();
 #pragma unroll
         for (int i = 0; i < MF; ++i) {
             const int u = R * MF + i;
@@ -415,9 +401,7 @@ struct Mm {
 #pragma unroll
                 for (int v = kUses - kD; v < kSync; ++v) a[v % kD] = frag_at(ot, (v + kD - kUses) / MF, (v + kD - kUses) % MF);
             }
-#pragma unroll
-            for (int f = 0; f < NF; ++f)
-                acc[f][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bc[f], a[u % kD], acc[f][i], 0, 0, 0);
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[R & 1], a[u % kD], acc[i], 0, 0, 0);
             if (u + kD < kUses)
                 a[u % kD] = frag_at(st, (u + kD) / MF, (u + kD) % MF);
             else if (u >= kSync)
@@ -453,7 +437,7 @@ struct Mm {
         lds_barrier();
 #pragma unroll
         for (int u = 0; u < kD; ++u) a[u] = frag_at(s0, u / MF, u % MF);
-        make_b<0, 0>(b[0]);
+        b[0] = make_b<0, 0>();
         for (uint32_t kb = kb0; kb < kb1; ++kb) {
             // the last super-block loads and stages itself again
             const uint32_t kn = kb + 1 < kb1 ? kb + 1 : kb;
@@ -465,33 +449,32 @@ struct Mm {
     }
 };
 
-// D (weights as the A operand): register 4q + j of fragment (f, i) holds X row
-// wm*MF*32 + i*32 + lane%32 and weight row f*32 + 8q + 4kh + j of the wave's, so
-// a lane's groups of four values are consecutive output columns.
-template <int FMT, int MF, int NF, int WM, int WN, bool SWIGLU>
+// D (weights as the A operand): register 4q + j of fragment i holds X row i*32 +
+// lane%32 and weight row 8q + 4kh + j of the wave's, so a lane's groups of four
+// values are consecutive output columns.
+template <int FMT, int MF, int WN, bool SWIGLU>
 __device__ __forceinline__ void mm_body(const PfGemm& p, uint32_t tile, uint8_t* s0, uint8_t* s1)
 {
-    using T = Mm<FMT, MF, NF, WM, WN>;
+    using T = Mm<FMT, MF, WN>;
     static_assert(!SWIGLU || WN % 2 == 0, "gate and up waves");
     T t;
     t.init_x(p);
-    const uint32_t l31 = threadIdx.x & 31u, wn = t.wave % WN, wm = t.wave / WN;
-    constexpr int kCols = SWIGLU ? NF * 32 * WN / 2 : NF * 32 * WN;  // output columns of the tile
-    const bool up = SWIGLU && wn >= WN / 2;
-    const uint32_t c0 = (SWIGLU ? wn % (WN / 2) : wn) * (NF * 32u);  // the wave's first column in the tile
+    const uint32_t l31 = threadIdx.x & 31u;
+    constexpr int kCols = SWIGLU ? 16 * WN : 32 * WN;  // output columns of the tile
+    const bool up = SWIGLU && t.wave >= WN / 2;
+    const uint32_t c0 = (SWIGLU ? t.wave % (WN / 2) : t.wave) * 32u;  // the wave's first column in the tile
     const uint32_t kb0 = SWIGLU ? 0u : blockIdx.y * p.bps, kb1 = SWIGLU ? p.nb : min(p.nb, kb0 + p.bps);
     const uint32_t row0 = tile * kCols;  // < N
     // the wave's own weight rows (past N: the last row again), so that 32-bit
     // offsets reach every K that the host lets through
-    const uint32_t first = min(row0 + c0, p.N - 1u), rows = min(p.N - first, NF * 32u);
+    const uint32_t first = min(row0 + c0, p.N - 1u), rows = min(p.N - first, 32u);
     t.wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(up ? p.w1 : p.w0) + uint64_t(first) * p.row_bytes, (short)0,
                                              int(rows * uint32_t(p.row_bytes)), 0x00020000);
-#pragma unroll
-    for (int f = 0; f < NF; ++f) t.wrow[f] = min(f * 32u + l31, rows - 1u) * uint32_t(p.row_bytes);
+    t.wrow = min(l31, rows - 1u) * uint32_t(p.row_bytes);
     t.run(s0, s1, kb0, kb1);
 
-    auto quad = [&](int f, int i, int q) {
-        return f32x4{t.acc[f][i][4 * q], t.acc[f][i][4 * q + 1], t.acc[f][i][4 * q + 2], t.acc[f][i][4 * q + 3]};
+    auto quad = [&](int i, int q) {
+        return f32x4{t.acc[i][4 * q], t.acc[i][4 * q + 1], t.acc[i][4 * q + 2], t.acc[i][4 * q + 3]};
     };
     if constexpr (SWIGLU) {
         // Gate values go to stage 0, up values to stage 1 ([row][column] fp32, 32
@@ -509,90 +492,83 @@ __device__ __forceinline__ void mm_body(const PfGemm& p, uint32_t tile, uint8_t*
         const float* sg = reinterpret_cast<const float*>(s0);
         const float* su = reinterpret_cast<const float*>(s1);
 #pragma unroll
-        for (int ib = 0; ib < MF; ib += kI)
-            for (uint32_t half = 0; half < uint32_t(WM); ++half) {
-                if (wm == half)
+        for (int ib = 0; ib < MF; ib += kI) {
 #pragma unroll
-                    for (int f = 0; f < NF; ++f)
+            for (int i = 0; i < kI; ++i)
 #pragma unroll
-                        for (int i = 0; i < kI; ++i)
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<f32x4*>(mine + (i * 32 + l31) * kLd + c0 + 8 * q + 4 * t.kh) = quad(ib + i, q);
+            __syncthreads();
+            for (uint32_t e = threadIdx.x; e < uint32_t(kI * 32 * kPieces); e += 64 * WN) {
+                const uint32_t r = e / kPieces, c = (e % kPieces) * 8u;
+                const uint32_t m = ib * 32u + r, col = tile * kCols + c;
+                if (m >= p.M || col >= p.N) continue;
+                half8 o;
 #pragma unroll
-                            for (int q = 0; q < 4; ++q)
-                                *reinterpret_cast<f32x4*>(mine + (i * 32 + l31) * kLd + c0 + f * 32 + 8 * q + 4 * t.kh) =
-                                    quad(f, ib + i, q);
-                __syncthreads();
-                for (uint32_t e = threadIdx.x; e < uint32_t(kI * 32 * kPieces); e += 64 * WM * WN) {
-                    const uint32_t r = e / kPieces, c = (e % kPieces) * 8u;
-                    const uint32_t m = half * (MF * 32u) + ib * 32u + r, col = tile * kCols + c;
-                    if (m >= p.M || col >= p.N) continue;
-                    half8 o;
+                for (int q = 0; q < 2; ++q) {
+                    const f32x4 gv = *reinterpret_cast<const f32x4*>(sg + r * kLd + c + 4 * q);
+                    const f32x4 uv = *reinterpret_cast<const f32x4*>(su + r * kLd + c + 4 * q);
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        const f32x4 gv = *reinterpret_cast<const f32x4*>(sg + r * kLd + c + 4 * q);
-                        const f32x4 uv = *reinterpret_cast<const f32x4*>(su + r * kLd + c + 4 * q);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) o[4 * q + j] = _Float16(mm_silu(gv[j]) * uv[j]);
-                    }
-                    _Float16* dst = p.s + uint64_t(m) * p.lds_out + col;
-                    if (vec && col + 8u <= p.N) {
-                        *reinterpret_cast<half8*>(dst) = o;
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 8; ++j)
-                            if (col + j < p.N) dst[j] = o[j];
-                    }
+                    for (int j = 0; j < 4; ++j) o[4 * q + j] = _Float16(mm_silu(gv[j]) * uv[j]);
                 }
-                __syncthreads();
+                _Float16* dst = p.s + uint64_t(m) * p.lds_out + col;
+                if (vec && col + 8u <= p.N) {
+                    *reinterpret_cast<half8*>(dst) = o;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if (col + j < p.N) dst[j] = o[j];
+                }
             }
+            __syncthreads();
+        }
     } else {
         const bool vec = (p.ldo & 3u) == 0;  // the partial buffer is 16-byte aligned
 #pragma unroll
         for (int i = 0; i < MF; ++i) {
-            const uint32_t m = wm * (MF * 32u) + i * 32u + l31;
+            const uint32_t m = i * 32u + l31;
             if (m >= p.M) continue;
             float* o = p.out + (uint64_t(blockIdx.y) * p.mpad + m) * p.ldo;
 #pragma unroll
-            for (int f = 0; f < NF; ++f)
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t col = row0 + c0 + 8u * q + 4u * t.kh;
+                if (vec && col + 4u <= p.N) {
+                    *reinterpret_cast<f32x4*>(o + col) = quad(i, q);
+                } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t col = row0 + c0 + f * 32u + 8u * q + 4u * t.kh;
-                    if (vec && col + 4u <= p.N) {
-                        *reinterpret_cast<f32x4*>(o + col) = quad(f, i, q);
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            if (col + j < p.N) o[col + j] = t.acc[f][i][4 * q + j];
-                    }
+                    for (int j = 0; j < 4; ++j)
+                        if (col + j < p.N) o[col + j] = t.acc[i][4 * q + j];
                 }
+            }
         }
     }
 }
 
-template <int FMT, int MF, int NF, int WM, int WN, bool SWIGLU>
-__global__ __launch_bounds__(64 * WM * WN, 1) void k_mm(PfGemm p)
+template <int FMT, int MF, int WN, bool SWIGLU>
+__global__ __launch_bounds__(64 * WN, 1) void k_mm(PfGemm p)
 {
-    using T = Mm<FMT, MF, NF, WM, WN>;
+    using T = Mm<FMT, MF, WN>;
     __shared__ __align__(1024) uint8_t s0[T::kStageB];
     __shared__ __align__(1024) uint8_t s1[T::kStageB];
-    mm_body<FMT, MF, NF, WM, WN, SWIGLU>(p, blockIdx.x, s0, s1);
+    mm_body<FMT, MF, WN, SWIGLU>(p, blockIdx.x, s0, s1);
 }
 
 // The q, k (Q4_K) and v (format VF) projections of one layer in one launch:
 // q's column tiles, then k's, then v's; all write split partials into one
 // [split][mpad][hidden + 2*kv_dim] buffer.
-template <int VF, int MF, int NF, int WM, int WN>
-__global__ __launch_bounds__(64 * WM * WN, 1) void k_mm_qkv(PfGemm q, PfGemm k, PfGemm v)
+template <int VF, int MF, int WN>
+__global__ __launch_bounds__(64 * WN, 1) void k_mm_qkv(PfGemm q, PfGemm k, PfGemm v)
 {
-    using T = Mm<kFmtQ4, MF, NF, WM, WN>;
+    using T = Mm<kFmtQ4, MF, WN>;
     __shared__ __align__(1024) uint8_t s0[T::kStageB];
     __shared__ __align__(1024) uint8_t s1[T::kStageB];
     const uint32_t t = blockIdx.x;
     if (t < q.tiles)
-        mm_body<kFmtQ4, MF, NF, WM, WN, false>(q, t, s0, s1);
+        mm_body<kFmtQ4, MF, WN, false>(q, t, s0, s1);
     else if (t < q.tiles + k.tiles)
-        mm_body<kFmtQ4, MF, NF, WM, WN, false>(k, t - q.tiles, s0, s1);
+        mm_body<kFmtQ4, MF, WN, false>(k, t - q.tiles, s0, s1);
     else
-        mm_body<VF, MF, NF, WM, WN, false>(v, t - q.tiles - k.tiles, s0, s1);
+        mm_body<VF, MF, WN, false>(v, t - q.tiles - k.tiles, s0, s1);
 }
 
 }  // namespace arc

@@ -26,8 +26,6 @@
 
 namespace arc {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 // --------------------------------------------------------- small kernels
 // H[m] = dequant(token_embd[tokens[m]]); grid (nb, M), element formula of
 // the decode embedding.
@@ -571,7 +569,7 @@ template <int FMT, int MF, int WN, bool SW>
 hipError_t launch_mm_t(const PfGemm& p, uint32_t splits, hipStream_t st)
 {
     constexpr uint32_t cols = SW ? 16u * WN : 32u * WN;
-    hipLaunchKernelGGL((k_mm<FMT, MF, 1, 1, WN, SW>), dim3((p.N + cols - 1) / cols, splits), dim3(64 * WN), 0, st, p);
+    hipLaunchKernelGGL((k_mm<FMT, MF, WN, SW>), dim3((p.N + cols - 1) / cols, splits), dim3(64 * WN), 0, st, p);
     return hipGetLastError();
 }
 
@@ -598,7 +596,7 @@ hipError_t launch_gemm(int qtype, const PfGemm& p, uint32_t splits, hipStream_t 
 template <int VF, int MF>
 hipError_t launch_qkv_t(const PfGemm& q, const PfGemm& k, const PfGemm& v, uint32_t splits, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_mm_qkv<VF, MF, 1, 1, 4>), dim3(q.tiles + k.tiles + v.tiles, splits), dim3(256), 0, st, q, k, v);
+    hipLaunchKernelGGL((k_mm_qkv<VF, MF, 4>), dim3(q.tiles + k.tiles + v.tiles, splits), dim3(256), 0, st, q, k, v);
     return hipGetLastError();
 }
 
