@@ -2,7 +2,9 @@
 MFMA projection GEMMs against the fp64 oracle, per element at the GEMV bar
 (|gpu - ref| <= 1e-3 * max(|ref|, 1e-3 * max|ref|)).
 
-Attention (arc_attention_decode: the decode step's kernel and split plan):
+Attention (arc_attention_decode: the decode step's kernel; past 2048 positions
+the call picks its own launch shape, and the decode step's, 4 waves and one chunk
+per split at least, is tested beside it):
 oracle orc_attention_decode_f64, the restatement of
 src/arcllm_v1_i001r_p8c_profile_runtime.cpp:1177-1212
 (shaders/p7_attention_kv_online.comp), over the same fp16 caches, at
@@ -71,11 +73,12 @@ def test_attention_decode_vs_fp64(kv_cache, T, qscale):
     assert err <= TOL
 
 
-@pytest.mark.parametrize("waves,min_cps", [(8, 1), (4, 2), (8, 3)])
-@pytest.mark.parametrize("T", [1, 127, 128, 129, 511, 512, 513, 2048, 4096, 4097])
+@pytest.mark.parametrize("waves,min_cps", [(4, 1), (8, 1), (4, 2), (8, 2), (8, 3)])
+@pytest.mark.parametrize("T", [1, 127, 128, 129, 511, 512, 513, 2048, 2049, 4095, 4096, 4097])
 def test_attention_decode_launch_shapes_vs_fp64(kv_cache, T, waves, min_cps):
-    """The tuning launch shapes: 8 waves (128-position chunks) and several
-    chunks per split, against the fp64 attention (qscale 4)."""
+    """The launch shapes: the decode step's (4 waves, one chunk per split at
+    least), 8 waves (128-position chunks) and several chunks per split, against
+    the fp64 attention (qscale 4)."""
     max_ctx, kc, vc, dkc, dvc = kv_cache
     q = (arc.synth_normal(SEED, 20 + T, KVH * HPK * 128) * 4.0).astype(np.float32)
     out = arc.DeviceBuffer(q.nbytes)
