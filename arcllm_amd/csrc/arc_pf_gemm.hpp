@@ -285,6 +285,14 @@ __device__ __forceinline__ void lds_barrier()
 
 typedef __attribute__((address_space(3))) void lds_void;
 
+// The largest divisor of n that is at most `most`.
+constexpr int mm_divisor(int n, int most)
+{
+    int d = most < n ? most : n;
+    while (n % d) --d;
+    return d;
+}
+
 template <int FMT, int MF, int WN>
 struct Mm {
     static constexpr int kRows = 32 * MF;                // X rows of the tile
@@ -484,8 +492,8 @@ __device__ __forceinline__ void mm_body(const PfGemm& p, uint32_t tile, uint8_t*
         // launch's fixed cost to 23 us.
         constexpr int kLd = 32 * (kCols + 4) * 4 <= T::kStageB ? kCols + 4 : kCols;
         constexpr int kFit = T::kStageB / (32 * kLd * 4);
-        constexpr int kI = kFit >= MF ? MF : kFit >= 4 ? 4 : kFit >= 2 ? 2 : 1;  // fragments per round
-        static_assert(kFit >= 1 && MF % kI == 0, "a fragment fits a stage");
+        static_assert(kFit >= 1, "a fragment fits a stage");
+        constexpr int kI = mm_divisor(MF, kFit);  // fragments per round
         constexpr int kPieces = kCols / 8;
         const bool vec = ((reinterpret_cast<uintptr_t>(p.s) | (p.lds_out * 2u)) & 15u) == 0;
         float* mine = reinterpret_cast<float*>(up ? s1 : s0);

@@ -558,9 +558,14 @@ thread_local int g_pf_attn_mfma = 1;  // 0: the VALU attention kernel (k_pf_attn
 // 32) and 32 weight rows, so each weight is decoded once.  Plain products take
 // 4 waves (128 weight rows; 256 workgroups of them ran 17 % faster than 128 of
 // 8 waves, 3.7 against 4.3 us per super-block at 256 rows), split over K to
-// about one workgroup per CU; the fused gate/up, not split, 8 past 64 rows (128
-// gate and 128 up rows: 148 workgroups for 18944 columns, where 4 waves would
-// leave 40 CUs with a second one).
+// about one workgroup per CU.  The fused gate/up, not split, takes 4 waves (64
+// gate and 64 up rows) while that gives no CU a second workgroup, and 8 (128 and
+// 128) for more columns and more than 64 rows; us, 4 waves / 8 waves:
+//   columns x K     65 rows       100 rows      192 rows      256 rows
+//    1024 x 2048  15.2 / 22.0   17.1 / 25.5   23.9 / 36.0   28.6 / 44.6
+//    8192 x 3584  23.1 / 33.7   26.0 / 38.9   37.3 / 55.3   44.5 / 69.4
+//   14336 x 4096  29.8 / 38.5   35.3 / 44.4   51.5 / 63.1   64.5 / 78.8
+//   18944 x 3584  38.2 / 34.7   47.2 / 42.0   81.3 / 60.6  101.2 / 76.0  (64 rows: 32.0 / 30.9)
 #define ARC_MM_ROWS(M, CALL) \
     ((M) > 192 ? CALL(8) : (M) > 128 ? CALL(6) : (M) > 96 ? CALL(4) : (M) > 64 ? CALL(3) : (M) > 32 ? CALL(2) : CALL(1))
 constexpr uint32_t kMmCols = 128;  // weight rows per workgroup of a plain product
@@ -575,7 +580,8 @@ hipError_t launch_mm_t(const PfGemm& p, uint32_t splits, hipStream_t st)
 
 hipError_t launch_gateup(const PfGemm& p, hipStream_t st)
 {
-#define ARC_MM_CALL(MF) (launch_mm_t<kFmtQ4, MF, (MF >= 3 ? 8 : 4), true>(p, 1, st))
+#define ARC_MM_CALL(MF) (wide ? launch_mm_t<kFmtQ4, MF, (MF >= 3 ? 8 : 4), true>(p, 1, st) : launch_mm_t<kFmtQ4, MF, 4, true>(p, 1, st))
+    const bool wide = p.N > 64u * kPfTargetWgs;
     return ARC_MM_ROWS(p.M, ARC_MM_CALL);
 #undef ARC_MM_CALL
 }

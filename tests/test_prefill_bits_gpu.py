@@ -93,6 +93,7 @@ PINNED = [
     (qkv, (arc.Q6_K_PADDED, 512, 256, 1024, 150), "7fa4f3692e91c8f8"),
     (gateup, (200, 1024, 100), "bc1cdfbaf041a142"),
     (gateup, (2048, 512, 256), "f39bd34dfea392e2"),
+    (gateup, (16400, 512, 180), "9de6f393c58c9446"),
     (attention, (2, 7, 300, 70, True), "a2fb4329a706cae2"),
     (attention, (3, 2, 0, 256, True), "e52f36b1b0bf8257"),
     (attention, (2, 7, 300, 70, False), "c5b278c8ae9a2993"),

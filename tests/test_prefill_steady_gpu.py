@@ -106,6 +106,25 @@ def test_gateup(weights, M):
         assert orc.rel_err(got[m], ref) <= TOL, m
 
 
+@pytest.mark.parametrize("N", [16384, 16385, 16500])  # past 16384 columns and 64 rows: 8 waves
+@pytest.mark.parametrize("M", [64, 65, 96, 100, 150, 200, 256])
+def test_gateup_wide(weights, N, M):
+    K = 768
+    wg, dg, _ = weights(arc.Q4_K, N, K, 11)
+    wu, du, _ = weights(arc.Q4_K, N, K, 12)
+    x = x16(M, K, 900 + M, 0.05)
+    s, ws = arc.DeviceBuffer((M * N + 64) * 2), arc.DeviceBuffer(arc.prefill_gemm_workspace_bytes(N, K))
+    s.zero()
+    arc.prefill_gateup(dg, du, N, K, dev(x.view(np.uint16)), M, s, ws)
+    out = s.download(np.uint16)
+    got = out[:M * N].view(np.float16).reshape(M, N).astype(np.float64)
+    for m in some(M):
+        xm = x[m].astype(np.float64)
+        ref = orc.swiglu_f64(orc.gemv_r64_f16(arc.Q4_K, wg, N, K, xm), orc.gemv_r64_f16(arc.Q4_K, wu, N, K, xm))
+        assert orc.rel_err(got[m], ref) <= TOL, m
+    assert not out[M * N:].any(), "wrote past the result"
+
+
 def q4_f64(w):
     """The exact weights of Q4_K blocks, [blocks, 256] in float64."""
     b = w.reshape(-1, 144)
