@@ -21,30 +21,32 @@
 //
 // What bounds it: instruction issue, and at full size the chip's power (a
 // library fp16 product of 8192^3 runs at 1.23 PFLOP/s on this card, one of 256 x
-// 37888 x 3584 without any decoding at 0.93).  A 32x32x16 MFMA takes 32 cycles
+// 37888 x 3584 without any decoding at 0.94).  A 32x32x16 MFMA takes 32 cycles
 // and two of their eight issue slots, so six other vector instructions are free
-// with two waves per SIMD (a 16x16x32 one takes 16 cycles and leaves two); the
-// decode costs 2.25 per weight (0.75 to mask the codes, v_fma_mix_f32, half a
-// v_cvt_pk_f16_f32).  Each wave takes all rows of the pass, so a weight
-// is decoded once and feeds up to 8 MFMAs: 2.4 other vector instructions and
-// one LDS read (4 cycles of the LDS) per MFMA.  Gate/up 18944 x 3584 at 256 rows
-// (whole call): 76 us, 917 TFLOP/s, 100 us before (34 instructions to decode 8
+// with two waves per SIMD (a 16x16x32 one takes 16 cycles and leaves two).  The
+// loop spends 2.59 per Q4_K weight (0.75 to mask the codes, v_fma_mix_f32, half a
+// v_cvt_pk_f16_f32, the rest factors, scales and addresses) and 3.70 per Q6_K
+// weight.  Each wave takes all rows of the pass, so a weight is decoded once and
+// feeds up to 8 MFMAs: as many other vector instructions and one LDS read (4
+// cycles of the LDS) per MFMA.  Whole calls, before (34 instructions to decode 8
 // weights, X through registers, two barriers' skew per super-block, a 30 KB
-// epilogue); at 100 rows 42 against 62; down 3584 x 18944 57 against 69; q|k|v at
-// 23 rows 12.6 against 18.6.  The weights are loaded 12 steps ahead: with 8 (and
-// waited for together with X) weights from HBM cost 10 us more than weights from
-// the Infinity Cache (gate/up 89 against 79 us).  Tiles measured for the gate/up kernel alone: 32 x
-// 256 per wave, 8 waves 76-78 us; 64 x 128 (each weight decoded twice) 87; 48 x 128
-// and 48 x 256 with 16x16x32 77-78, 80 x 128 in 4 waves 78.
+// epilogue) and now: gate/up 18944 x 3584 at 256 rows 100 / 78 us (890 TFLOP/s), at
+// 100 rows 62 / 43; down 3584 x 18944 69 / 55; q|k|v at 23 rows 18.6 / 12.5.
+// The weights are loaded 12 steps ahead: with 8 (and waited for together with X)
+// weights from HBM cost 10 us more than weights from the Infinity Cache (gate/up at
+// 256 rows); now 81.4 us over ten sets of weights in turn, 80.7 over one.  Inside a
+// prompt the launch still takes 8 us longer (88.9 traced), the weights being no
+// reason for it.  Tiles measured for the gate/up kernel alone: 32 x 256 per wave, 8
+// waves 76-78 us; 64 x 128 (each weight decoded twice) 87; 48 x 128 and 48 x 256 with
+// 16x16x32 77-78, 80 x 128 in 4 waves 78.
 //
 // X goes from global memory straight into LDS (16 bytes per lane, no
 // registers), half a super-block (128 columns) per stage, two stages.  A stage's
 // row is 256 bytes; its 16-byte pieces are stored at piece ^ (row % 16), so 16
 // consecutive rows of a fragment read lie in 16 different bank groups.
-// One barrier per stage, in the middle of its last step: by then every wave
-// holds the last step's fragments in registers, so the barrier both frees the
-// stage for the next fill and publishes the other one, whose first fragments
-// are read behind the second half of the step's MFMAs.
+// One barrier per stage, two fragments before its end: by then every wave holds
+// those in registers, so the barrier both frees the stage for the next fill and
+// publishes the other one, whose first fragments are read behind the MFMAs left.
 #pragma once
 
 #include "arc_device.hpp"

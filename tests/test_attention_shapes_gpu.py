@@ -1,6 +1,6 @@
 """arc_attention_decode picks its launch shape (waves per workgroup, chunks per
-split) from the context length: the contexts on both sides of each line, few
-and many kv heads, against fp64 (per element 1e-3, the bar of the kernel) and
+split) from the context length and the kv heads: the contexts on both sides of
+each line, few and many kv heads, against fp64 (per element 1e-3, the bar of the kernel) and
 against the shape of short contexts.  Two shapes differ only in the order of
 fp32 sums of at most 6001 terms with weights that sum to 1: relative to the
 largest output below 6001 * 2^-24 = 3.6e-4 at worst, some 1e-6 measured."""
