@@ -512,7 +512,13 @@ static bool attn_eight_waves(uint32_t T, uint32_t kv_heads)
 
 // Sets ap.min_cps and launches.  T = 0: the position is only known on the
 // device (grid kMaxSplits x kv heads; workgroups past its plan return at once).
-// Otherwise the grid is the plan's, and attn_eight_waves picks the shape.
+// Otherwise attn_eight_waves picks the shape, and the grid is the plan's where the
+// idle workgroups cost time: from 5 kv heads on, up to the 768 workgroups of 4 waves
+// that the CUs hold.  Elsewhere the full grid is as fast or faster, as it keeps split
+// s of every kv head on XCD s % 8.  us, full grid / the plan's:
+//   2x4 T = 300   7.8 /  8.1   2x4 T = 800  8.5 /  8.7   1x8 T = 500  9.35 / 9.5   4x7 T = 65  9.07 / 9.19
+//   6x5 T = 300  10.2 /  8.8   8x8 T = 1024 12.8 / 11.0  32x2 T = 500 13.9 / 9.1
+//  32x2 T = 1500 (768 workgroups) 16.7 / 15.2   T = 2048 (1024) 18.7 / 19.5
 static void launch_attn(AttnParams ap, uint32_t kv_heads, hipStream_t st, uint32_t T = 0)
 {
     int waves = g_attn_waves ? g_attn_waves : 4;
@@ -521,7 +527,11 @@ static void launch_attn(AttnParams ap, uint32_t kv_heads, hipStream_t st, uint32
         waves = 8;
         ap.min_cps = T > 4096 ? 2u : 1u;
     }
-    const uint32_t nsplit = T ? attn_split(T, uint32_t(waves) * kAttnTile, ap.min_cps).nsplit : uint32_t(kMaxSplits);
+    uint32_t nsplit = kMaxSplits;
+    if (T) {
+        const uint32_t plan = attn_split(T, uint32_t(waves) * kAttnTile, ap.min_cps).nsplit;
+        if (waves == 8 || (kv_heads > 4 && plan * kv_heads <= 768)) nsplit = plan;
+    }
     if (waves == 8)
         launch_attn_w<8>(ap, nsplit, kv_heads, st);
     else

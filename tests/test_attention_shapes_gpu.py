@@ -75,3 +75,19 @@ def test_rule(kv_heads, hpk, T, shape):
         assert np.array_equal(got[0, 0], got[tune]) == (tune == shape), tune
     ref = orc.attention_decode_f64(q, kc, vc, T, kv_heads * hpk, kv_heads)
     assert orc.rel_err(got[0, 0].view(np.float32), ref) <= 1e-3
+
+
+# the full grid of 64 splits and the plan's, on both sides of 4 kv heads and of 768 workgroups
+@pytest.mark.parametrize("kv_heads,hpk,T", [(4, 1, 1), (5, 1, 1), (4, 7, 300), (5, 7, 300), (32, 2, 1536), (32, 2, 1537)])
+def test_grid(kv_heads, hpk, T):
+    n = kv_heads * hpk * 128
+    kc = arc.synth_normal(SEED, 21, T * kv_heads * 128).astype(np.float16)
+    vc = arc.synth_normal(SEED, 22, T * kv_heads * 128).astype(np.float16)
+    q = arc.synth_normal(SEED, 23, n) * np.float32(2.0)
+    out, ws = arc.DeviceBuffer(n * 4), arc.DeviceBuffer(arc.attention_workspace_bytes(kv_heads, hpk))
+    got = []
+    for _ in range(3):  # the workspace keeps what the call before left
+        arc.attention_decode(dev(q), dev(kc), dev(vc), kv_heads, hpk, T, T, out, ws)
+        got.append(out.download(np.float32))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    assert orc.rel_err(got[0], orc.attention_decode_f64(q, kc, vc, T, kv_heads * hpk, kv_heads)) <= 1e-3
